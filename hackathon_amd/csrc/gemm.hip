@@ -136,6 +136,7 @@ int c3h_conv2d(const c3h_conv_args* a, void* stream) {
     p.fd_kwpack = make_fastdiv(static_cast<uint32_t>(p.kw_pack));
     p.k = static_cast<int64_t>(a->kh) * a->kw * a->c_pack;
     p.ldb = p.k;
+    p.b_bytes = static_cast<int64_t>(a->o) * p.ldb * 4;
     bool handled = false;
     rc = launch_conv_direct_c4(p, s, &handled);  // 4-channel inputs: direct VALU conv
     if (handled) return rc;

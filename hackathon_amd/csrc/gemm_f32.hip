@@ -101,7 +101,41 @@ int launch_conv_direct_c4(Problem p, hipStream_t s, bool* handled) {
   return launch_status("conv_direct_c4");
 }
 
+namespace {
+
+// fp32 on the direct-to-LDS pipeline: 64 x 64 tiles, wave tiles 16 x 64, the
+// next K tile's fragments read into a second register set under the current
+// one's MFMAs (mfma_gemm_dma_kernel, RP).  Bound by the fp32 MFMA (a K tile
+// is 1024 MFMA cycles per CU against 16 KB of DMA), so the small tile costs
+// nothing in operand traffic: 128 x 128, 128 x 64 and 256 x 64 tiles and
+// three or four stages measured equal or slower on every shape tried, and
+// 64 x 64 leaves the fewest CUs idle.  Against the register-staged kernel
+// below (its k-major LDS tiles took four scalar LDS stores per load and a
+// scalar read per MFMA operand): 3x3 convs of a batch of 256, 128 channels
+// 16 x 16 220 -> 157 us (123 TFLOP/s; a pure MFMA loop reaches 151), 512
+// channels 4 x 4 274 -> 169 us; dense 2048 x 2048 x 512 75 -> 40 us,
+// 2048 x 512 x 512 28 -> 15 us.
+template <int AM>
+int launch_f32_dma(Problem p, hipStream_t s) {
+  dim3 grid;
+  grid_of<64, 64>(p, 1, grid);
+  hipLaunchKernelGGL((mfma_gemm_dma_kernel<MmaF32, float, 64, 64, 4, 1, AM, 2, 4, true>), grid, dim3(kThreads), 0, s,
+                     p);
+  return launch_status("gemm_f32");
+}
+
+}  // namespace
+
 int launch_f32_modes(Problem p, int64_t batch, hipStream_t s, int am, bool b_kcontig) {
+  // The pipeline moves whole 16-byte chunks along K (k % 4 == 0; rows are
+  // 16-byte aligned on every caller's path) at 32-bit byte offsets, and a
+  // conv's 32-wide K tile has to lie inside one filter tap.
+  constexpr int64_t kMaxBytes = int64_t{1} << 31;
+  if (batch == 1 && b_kcontig && p.k % 4 == 0 && p.a_bytes > 0 && p.a_bytes < kMaxBytes && p.b_bytes > 0 &&
+      p.b_bytes < kMaxBytes && !switches().disable_dma) {
+    if (am == kDenseK) return launch_f32_dma<kDenseK>(p, s);
+    if (am == kConv && p.c_pack % 32 == 0) return launch_f32_dma<kConvTap>(p, s);
+  }
   if (am == kDenseM) return b_kcontig ? launch_f32<kDenseM, true>(p, batch, s) : launch_f32<kDenseM, false>(p, batch, s);
   if (am == kDenseK) return b_kcontig ? launch_f32<kDenseK, true>(p, batch, s) : launch_f32<kDenseK, false>(p, batch, s);
   if (am == kConv) return launch_f32<kConv, true>(p, batch, s);

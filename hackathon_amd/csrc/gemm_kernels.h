@@ -5,7 +5,7 @@
 // instantiated in its own translation unit (gemm_<type>.hip), so they build
 // in parallel, and gemm.hip holds the C entry points.
 //
-//   fp32  : v_mfma_f32_16x16x4_f32   (configs 1-2, the reference's fp32 policy)
+//   fp32  : v_mfma_f32_16x16x4_f32   (the reference's fp32 policy)
 //   bf16  : v_mfma_f32_16x16x32_bf16 (config 3)
 //   f16   : v_mfma_f32_16x16x32_f16  (config 4)
 //
@@ -692,6 +692,40 @@ struct MmaF8 {
     return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, c, 0, 0, 0, 0, 0, 0);
   }
 };
+
+// fp32 (v_mfma_f32_16x16x4_f32).  A lane's operand vector is one 16-byte
+// chunk, k = 16 q + 4 g + e (e = 0..3) for K step q and lane group g, and
+// element e of every lane makes one 16x16x4 MFMA: K in steps of
+// {e, 4 + e, 8 + e, 12 + e}, the same for A and B.
+struct MmaF32 {
+  typedef f32x4 vec;
+  typedef f32x4 acc_t;
+  static constexpr int ES = 4;
+  static constexpr bool kInt = false;
+  static constexpr int kStep = 4;
+  static constexpr bool kScaled = false;
+};
+
+// One K step of a wave tile: acc[i][j] += bv[j] x av[i] (operands swapped,
+// C^T: see epilogue_direct).  fp32 walks the four MFMAs of a chunk outermost,
+// so that consecutive MFMAs go to different accumulators.
+template <typename Mma, int TM, int TN, typename Acc, typename Vec>
+__device__ __forceinline__ void mma_step(Acc (&acc)[TM][TN], const Vec (&av)[TM], const Vec (&bv)[TN]) {
+  if constexpr (std::is_same<Mma, MmaF32>::value) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bv[j][e], av[i][e], acc[i][j], 0, 0, 0);
+  } else {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) acc[i][j] = Mma::mma(bv[j], av[i], acc[i][j]);
+  }
+}
 
 // MFMA operand of tile row `r` (row base `row`, XOR-swizzled 16-byte chunks)
 // for the K step starting at chunk ks.
@@ -2214,7 +2248,7 @@ __global__ void __launch_bounds__(NW * 64) mfma_gemm_dma_kernel(Problem p) {
   } else if constexpr (RP) {
     static_assert(LPW * (S - 1) < 64, "vmcnt range");
     constexpr int KS = 8 / Mma::kStep;
-    constexpr int N_MFMA = KS * TM * TN;
+    constexpr int N_MFMA = KS * TM * TN * (std::is_same<Mma, MmaF32>::value ? 4 : 1);
     constexpr int N_DSR = KS * (TM + TN) * (Mma::kStep == 8 ? 2 : 1);
     constexpr int PER = N_MFMA / N_DSR;
     vec av[2][KS][TM], bv[2][KS][TN];
@@ -2262,11 +2296,7 @@ __global__ void __launch_bounds__(NW * 64) mfma_gemm_dma_kernel(Problem p) {
       // between every PER MFMAs of tile kt.
       read_frags(std::integral_constant<int, SET ^ 1>{}, static_cast<int>((kt + 1) % S));
 #pragma unroll
-      for (int q = 0; q < KS; ++q)
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-          for (int j = 0; j < TN; ++j) acc[i][j] = Mma::mma(bv[SET][q][j], av[SET][q][i], acc[i][j]);
+      for (int q = 0; q < KS; ++q) mma_step<Mma, TM, TN>(acc, av[SET][q], bv[SET][q]);
 #pragma unroll
       for (int g = 0; g < N_DSR; ++g) {
         __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);    // one LDS read
@@ -2326,13 +2356,7 @@ __global__ void __launch_bounds__(NW * 64) mfma_gemm_dma_kernel(Problem p) {
     // other waits on its DMA, barrier and LDS reads.
     if constexpr (kPrio) __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-    for (int q = 0; q < KS; ++q)
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) {
-          acc[i][j] = Mma::mma(bv[q][j], av[q][i], acc[i][j]);  // C^T: see epilogue_direct
-        }
+    for (int q = 0; q < KS; ++q) mma_step<Mma, TM, TN>(acc, av[q], bv[q]);
     if constexpr (kPrio) __builtin_amdgcn_s_setprio(0);
     __builtin_amdgcn_sched_barrier(0);
   }

@@ -1613,3 +1613,67 @@ def test_nonfinite_flag(gpu, kind):
                 y = x.copy()
                 y[pos] = bad
                 assert run(y) == 1, (n, pos, bad)
+
+
+@pytest.mark.parametrize("m,n,k,form", [(65, 68, 36, "relu"), (64, 64, 32, "plain"), (1024, 4, 4, "relu"),
+                                        (333, 200, 2048, "program"), (130, 516, 100, "gelu"), (96, 67, 64, "relu")])
+def test_gemm_fp32_pipeline_edges(gpu, m, n, k, form):
+    """fp32 GEMM on the direct-to-LDS pipeline: rows, columns and K at and past the 64 x 64 x 32 tile edges,
+    K of one chunk, unaligned output rows (n = 67), and each epilogue form, against float64.  An fp32 dot
+    product of K terms is within K 2^-24 of sum |a b|; the epilogue adds a few roundings of its values."""
+    from hackathon_amd import _lib
+    from hackathon_amd.c35 import engine as E
+    from hackathon_amd.device import DeviceArray
+    from scipy.special import erf
+
+    rng = np.random.default_rng(m + n + k)
+    a, b = (rng.standard_normal(s, dtype=np.float32) for s in ((m, k), (n, k)))
+    bias, res = rng.standard_normal(n, dtype=np.float32), rng.standard_normal((m, n), dtype=np.float32)
+    prog = [(_lib.EW_MUL, 0, 2, 0.0), (_lib.EW_ADD, 1, 0, 0.0)]
+    kw = {"relu": dict(act=1), "plain": {}, "gelu": dict(act=2, imm=[math.sqrt(2.0), 1.0, 0.5]),
+          "program": dict(program=prog, imm=[0.25])}[form]
+    out = DeviceArray.empty((m, n), np.float32)
+    ad, bd, biasd, resd = _dev(a), _dev(b), _dev(bias), _dev(res)
+    E.gemm(ad, bd, out, m, n, k, lda=k, ldb=k, ldo=n, trans_b=1, in_dtype=_lib.F32,
+           epi=E.epilogue(bias=biasd, bias_mode=2, residual=resd, **kw))
+    a64, b64 = a.astype(np.float64), b.astype(np.float64)
+    v = a64 @ b64.T + bias + res
+    size = np.abs(a64) @ np.abs(b64).T + np.abs(bias) + np.abs(res)
+    ref = {"relu": np.maximum(v, 0), "plain": v, "gelu": 0.5 * v * (1 + erf(v / math.sqrt(2.0))),
+           "program": 1.25 * v}[form]
+    # the GELU's slope is below 1.13 and its erf adds |x| 2^-22; the program scales by 1.25
+    bound = 1.25 * (k + 8) * 2.0 ** -24 * size + np.abs(v) * 2.0 ** -21
+    assert np.all(np.abs(out.get() - ref) <= bound)
+
+
+@pytest.mark.parametrize("n,h,w,c,o,ks,stride,nchw", [(2, 9, 7, 32, 64, 3, 1, 0), (1, 5, 5, 64, 72, 1, 2, 0),
+                                                     (3, 4, 4, 96, 40, 3, 2, 1), (1, 1, 1, 32, 4, 3, 1, 0)])
+def test_conv_fp32_pipeline_edges(gpu, n, h, w, c, o, ks, stride, nchw):
+    """fp32 convs whose channels are whole 32-wide K tiles (the pipeline's tap-uniform form): images smaller
+    than the filter, strides, ragged channel counts and both output layouts, against float64 (same bound)."""
+    from hackathon_amd import _lib
+    from hackathon_amd.device import DeviceArray
+
+    rng = np.random.default_rng(n + h + c + o)
+    pad = ks // 2
+    ho, wo = (h + 2 * pad - ks) // stride + 1, (w + 2 * pad - ks) // stride + 1
+    x, wt = rng.standard_normal((n, h, w, c), dtype=np.float32), rng.standard_normal((o, ks, ks, c), dtype=np.float32)
+    bias = rng.standard_normal(o, dtype=np.float32)
+    out = DeviceArray.empty((n, o, ho, wo) if nchw else (n, ho, wo, o), np.float32)
+    xd, wd, bd = _dev(x), _dev(wt), _dev(bias)
+    a = _lib.ConvArgs()
+    a.x, a.w, a.out = xd.ptr, wd.ptr, out.ptr
+    a.n, a.c, a.h, a.w_, a.c_stride, a.c_pack, a.o, a.kh, a.kw, a.sh, a.sw = n, c, h, w, c, c, o, ks, ks, stride, stride
+    a.pad_top, a.pad_left, a.dh, a.dw, a.ho, a.wo = pad, pad, 1, 1, ho, wo
+    a.out_layout, a.in_dtype, a.out_dtype = 1 - nchw, _lib.F32, _lib.F32
+    a.epi.alpha, a.epi.beta, a.epi.bias, a.epi.bias_mode, a.epi.act = 1.0, 1.0, bd.ptr, 2, 1
+    _lib.launch(a)
+    xp = np.zeros((n, h + 2 * pad, w + 2 * pad, c))
+    xp[:, pad:pad + h, pad:pad + w] = x
+    cols = np.stack([xp[:, i:i + stride * ho:stride, j:j + stride * wo:stride] for i in range(ks) for j in range(ks)], 3)
+    cols = cols[:, :ho, :wo].reshape(n * ho * wo, -1)
+    w64 = wt.reshape(o, -1).astype(np.float64)
+    ref = np.maximum(cols @ w64.T + bias, 0).reshape(n, ho, wo, o)
+    bound = ((cols.shape[1] + 8) * 2.0 ** -24 * (np.abs(cols) @ np.abs(w64).T + np.abs(bias))).reshape(n, ho, wo, o)
+    got = out.get().transpose(0, 2, 3, 1) if nchw else out.get()
+    assert np.all(np.abs(got - ref) <= bound)
