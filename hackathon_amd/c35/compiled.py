@@ -1106,10 +1106,10 @@ class CompiledPlan:
         out = self._new(out_shape, self._out_dtype(st.final))
         self._finish_residual(st, out)
         mm = code
-        if code == _lib.F32:
-            splits = self._splitk(m, n, k)
-        else:  # 16-bit: 128x128 tiles, K tiles of 64
-            splits = self._splitk(m, n, k, vec=64, tile=128, min_k=64)
+        # GEMMs with few output tiles run on small tiles that split K inside
+        # one launch (c3h_gemm).  Only a 16-bit output of a single 128 x 128
+        # tile is still split over two launches.
+        splits = self._splitk(m, n, k) if code != _lib.F32 and m <= 128 and n <= 128 else 1
         if splits > 1:
             self._gemm_splitk(node, a2, w, out, st, m, n, k, splits, alpha, beta, bmode, in_code=code)
             return
@@ -1127,11 +1127,11 @@ class CompiledPlan:
             self._note_row_max_site(st, out, m, n, alpha, beta, bmode)
         self.vals[st.final] = out
 
-    def _splitk(self, m: int, n: int, k: int, vec: int = 4, tile: int = 64, min_k: int = 32) -> int:
-        """K splits for a GEMM whose tile x tile output tiles cannot fill two
-        blocks per CU (fp32: 64x64 tiles; 16-bit: 128x128): the largest split
-        with K/split a multiple of `vec`, at least `min_k` deep, and at most
-        two blocks per CU in total (1 = no split)."""
+    def _splitk(self, m: int, n: int, k: int, vec: int = 64, tile: int = 128, min_k: int = 64) -> int:
+        """K splits for a 16-bit GEMM whose tile x tile output tiles cannot
+        fill two blocks per CU: the largest split with K/split a multiple of
+        `vec`, at least `min_k` deep, and at most two blocks per CU in total
+        (1 = no split)."""
         tiles = -(-m // tile) * -(-n // tile)
         target = 2 * self._cus
         if 2 * tiles > target or k < 128:

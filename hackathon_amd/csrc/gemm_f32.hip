@@ -133,8 +133,11 @@ int launch_f32_modes(Problem p, int64_t batch, hipStream_t s, int am, bool b_kco
   constexpr int64_t kMaxBytes = int64_t{1} << 31;
   if (batch == 1 && b_kcontig && p.k % 4 == 0 && p.a_bytes > 0 && p.a_bytes < kMaxBytes && p.b_bytes > 0 &&
       p.b_bytes < kMaxBytes && !switches().disable_dma) {
+    const bool tap = am == kConv && p.c_pack % 32 == 0;
+    const int tile = am == kDenseK || tap ? ks_tile(p, batch, device_cus()) : 0;
+    if (tile) return launch_ks_f32(p, s, tap ? kConvTap : kDenseK, tile);
     if (am == kDenseK) return launch_f32_dma<kDenseK>(p, s);
-    if (am == kConv && p.c_pack % 32 == 0) return launch_f32_dma<kConvTap>(p, s);
+    if (tap) return launch_f32_dma<kConvTap>(p, s);
   }
   if (am == kDenseM) return b_kcontig ? launch_f32<kDenseM, true>(p, batch, s) : launch_f32<kDenseM, false>(p, batch, s);
   if (am == kDenseK) return b_kcontig ? launch_f32<kDenseK, true>(p, batch, s) : launch_f32<kDenseK, false>(p, batch, s);

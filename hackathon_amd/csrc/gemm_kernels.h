@@ -2547,6 +2547,27 @@ inline int device_cus() {
   return cus;
 }
 
+// Whether the small-output kernel takes this GEMM or tap-uniform conv, and on
+// which tile (gemm_ks.h; 0 = no, 1 = 16 x 32, 2 = 32 x 32): outputs of at
+// most one 16 x 32 tile, or two 32 x 32 tiles, per CU.  Measured on 256 CUs
+// against the best shared-tile kernel (fp16, us): 333 x 512 x 2048 (M x N x
+// K) 5.8 against 12.2, 200 x 2304 x 768 (504 tiles of 32 x 32) 5.9 against
+// 7.4, 1000 x 512 x 2048 (512 tiles) 9.5 against 12.7; past the line 333 x
+// 2048 x 512 (704 tiles) 7.7 against 6.3.  16 x 32 over 32 x 32 where both
+// fit: 200 x 512 x 2048 5.1 against 5.8, in fp32 (MFMA-bound: twice the CUs)
+// 9.1 against 13.6.  Row-major outputs without the row_max side output only.
+inline int ks_tile(const Problem& p, int64_t batch, int cus) {
+  if (batch != 1 || p.out_nchw || p.epi.row_max != nullptr || switches().disable_dma || p.a_bytes <= 0 ||
+      p.b_bytes <= 0 || p.a_bytes >= (int64_t{1} << 31) || p.b_bytes >= (int64_t{1} << 31))
+    return 0;
+  if (ceil_div(p.m, 16) * ceil_div(p.n, 32) <= cus) return 1;
+  return ceil_div(p.m, 32) * ceil_div(p.n, 32) <= 2 * cus ? 2 : 0;
+}
+int launch_ks_16(Problem p, hipStream_t s, int in_dtype, int am, int tile);          // gemm_ks_16.hip
+int launch_ks_i8(Problem p, hipStream_t s, int mode, int out_dtype, int tile);       // gemm_ks_8.hip
+int launch_ks_f8(Problem p, hipStream_t s, int out_dtype, int tile);                 // gemm_ks_8.hip
+int launch_ks_f32(Problem p, hipStream_t s, int am, int tile);                       // gemm_ks_8.hip
+
 template <typename Mma, typename TO, int AM>
 int launch_mfma(Problem p, int64_t batch, hipStream_t s, const char* what) {
   dim3 grid;
@@ -2637,6 +2658,10 @@ int launch_mfma(Problem p, int64_t batch, hipStream_t s, const char* what) {
 // 16-bit inputs write either the same 16-bit type or fp32.
 template <typename Mma, typename T, int AM>
 int launch_h(Problem p, int64_t batch, hipStream_t s, int in_dtype) {
+  if constexpr (AM == kDenseK || AM == kConvTap) {
+    if (p.out_dtype == C3H_F32 || p.out_dtype == in_dtype)
+      if (const int tile = ks_tile(p, batch, device_cus())) return launch_ks_16(p, s, in_dtype, AM, tile);
+  }
   if (p.out_dtype == C3H_F32) return launch_mfma<Mma, float, AM>(p, batch, s, "gemm_h");
   if (p.out_dtype == in_dtype) return launch_mfma<Mma, T, AM>(p, batch, s, "gemm_h");
   return fail(C3H_EUNSUPPORTED, "gemm: 16-bit inputs write fp32 or the input dtype, not %d", p.out_dtype);
@@ -2652,6 +2677,7 @@ int launch_h_any(Problem p, int64_t batch, hipStream_t s, int in_dtype) {
 // else the register-prefetch kernel.
 template <typename TO>
 int launch_fp8(Problem p, hipStream_t s) {
+  if (const int tile = ks_tile(p, 1, device_cus())) return launch_ks_f8(p, s, p.out_dtype, tile);
   dim3 grid;
   if (dma_eligible(p, 1, kDenseK) && big_tile_wins(p, device_cus(), sizeof(TO), false)) {
     grid_of<256, 256>(p, 1, grid);

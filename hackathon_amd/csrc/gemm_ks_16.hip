@@ -1,0 +1,25 @@
+// bf16 / fp16 instantiations of the small-output GEMM and conv (see gemm_ks.h).
+#include "gemm_ks.h"
+
+namespace c3h {
+namespace gk {
+
+namespace {
+template <typename Mma, typename T>
+int launch_ks_type(Problem p, hipStream_t s, int am, int tile) {
+  const bool f32 = p.out_dtype == C3H_F32;
+  if (am == kConvTap)
+    return f32 ? launch_ks_tile<Mma, float, kConvTap>(p, s, tile, "conv_ks")
+               : launch_ks_tile<Mma, T, kConvTap>(p, s, tile, "conv_ks");
+  return f32 ? launch_ks_tile<Mma, float, kDenseK>(p, s, tile, "gemm_ks")
+             : launch_ks_tile<Mma, T, kDenseK>(p, s, tile, "gemm_ks");
+}
+}  // namespace
+
+int launch_ks_16(Problem p, hipStream_t s, int in_dtype, int am, int tile) {
+  return in_dtype == C3H_BF16 ? launch_ks_type<MmaBF16, bf16_t>(p, s, am, tile)
+                              : launch_ks_type<MmaF16, f16_t>(p, s, am, tile);
+}
+
+}  // namespace gk
+}  // namespace c3h

@@ -1677,3 +1677,96 @@ def test_conv_fp32_pipeline_edges(gpu, n, h, w, c, o, ks, stride, nchw):
     bound = ((cols.shape[1] + 8) * 2.0 ** -24 * (np.abs(cols) @ np.abs(w64).T + np.abs(bias))).reshape(n, ho, wo, o)
     got = out.get().transpose(0, 2, 3, 1) if nchw else out.get()
     assert np.all(np.abs(got - ref) <= bound)
+
+
+@pytest.mark.parametrize("kind", ["fp32", "fp16", "bf16", "fp8", "int8"])
+@pytest.mark.parametrize("m,n,k,ldo,form", [
+    (1, 10, 64, 10, "relu"), (17, 33, 144, 40, "program"), (16, 32, 2048, 32, "gelu"),   # 16 x 32 tiles
+    (515, 289, 272, 292, "relu"), (1000, 512, 1040, 512, "gelu")])                      # 32 x 32 tiles
+def test_small_output_gemm_matches_the_general_kernel(gpu, kind, m, n, k, ldo, form):
+    """GEMMs of few output tiles split K over the waves of a workgroup: one row, ragged edges, fewer K tiles
+    than waves, a partial last K tile and strided output rows, against the register-staged kernel
+    (C3H_DISABLE_DMA).  int8 codes are equal; a float dot product of K terms moves by at most K 2^-23 of
+    sum |a b| between two summation orders, plus the output type's rounding."""
+    from hackathon_amd import _lib
+    from hackathon_amd.c35 import engine as E
+    from hackathon_amd.device import DeviceArray
+
+    rng = np.random.default_rng(m + n + k)
+    if kind == "fp8":  # finite E4M3 codes of magnitudes up to 1.875
+        a, b = (rng.integers(0, 0x40, s, dtype=np.uint8) | (rng.integers(0, 2, s, dtype=np.uint8) << 7) for s in
+                ((m, k), (n, k)))
+        size, out_np = 2.0 ** 2 * k * np.ones((m, n)), np.float16
+    elif kind == "int8":
+        a, b = (rng.integers(-128, 128, s, dtype=np.int8) for s in ((m, k), (n, k)))
+        out_np = np.int8
+    else:
+        (a, af), (b, bf) = ((x, x) if kind == "fp32" else _bits(x, kind) for x in
+                            (rng.standard_normal(s, dtype=np.float32) for s in ((m, k), (n, k))))
+        size, out_np = np.abs(af).astype(np.float64) @ np.abs(bf).T.astype(np.float64), a.dtype
+    bias, scale = _dev(rng.standard_normal(n, dtype=np.float32)), _dev(rng.random(max(m, n), dtype=np.float32) + 0.5)
+    prog = [(_lib.EW_MUL, 0, 2, 0.0), (_lib.EW_ADD, 1, 0, 0.0)]
+    epi = E.epilogue(bias=bias, bias_mode=2, **{"relu": dict(act=1), "gelu": dict(act=2, imm=[math.sqrt(2.0), 1.0, 0.5]),
+                                                "program": dict(program=prog, imm=[0.25])}[form])
+    ad, bd = _dev(a), _dev(b)
+
+    def run():
+        out = DeviceArray.from_host(np.zeros((m, ldo), out_np))
+        g = {"fp8": _lib.Fp8GemmArgs, "int8": _lib.QGemmArgs}.get(kind, _lib.GemmArgs)()
+        g.a, g.b, g.out, g.m, g.n, g.k, g.lda, g.ldb, g.ldo = ad.ptr, bd.ptr, out.ptr, m, n, k, k, k, ldo
+        g.epi = epi
+        if kind == "fp8":
+            g.a_scale, g.b_scale, g.out_dtype = scale.ptr, scale.ptr, _lib.F16
+        elif kind == "int8":
+            g.a_scale, g.y_scale, g.b_scale, g.mode, g.out_dtype = 0.002, 0.9, scale.ptr, 3, _lib.I8
+            g.act_dtype, g.q_scale, g.q_zero = _lib.BF16, 0.7, 3
+        else:
+            g.batch, g.trans_b, g.in_dtype, g.out_dtype = 1, 1, ad.code, ad.code
+        _lib.launch(g)
+        return out.get()
+
+    got, want = run(), switches.with_switch("C3H_DISABLE_DMA", "1", run)
+    if kind == "int8":
+        np.testing.assert_array_equal(got, want)
+        return
+    got, want = (x if kind in ("fp32", "fp8") else _from16(x, kind) for x in (got, want))
+    got, want = got.astype(np.float64), want.astype(np.float64)
+    assert not got[:, n:].any()
+    # slopes of the epilogue forms are at most 1.25; row and column scales of fp8 at most 1.5 each
+    bound = 1.25 * (2.25 if kind == "fp8" else 1.0) * k * 2.0 ** -23 * size
+    ulp = {"fp32": 2.0 ** -22, "bf16": 2.0 ** -7}.get(kind, 2.0 ** -10)
+    assert np.all(np.abs(got - want)[:, :n] <= bound + ulp * np.abs(want[:, :n]) + 2.0 ** -24)
+
+
+@pytest.mark.parametrize("kind,c", [("fp32", 32), ("bf16", 64), ("fp16", 192)])
+@pytest.mark.parametrize("n,hw,o,ks,stride", [(1, 7, 72, 3, 1), (2, 5, 512, 1, 2), (3, 14, 100, 3, 2)])
+def test_small_output_conv_matches_the_general_kernel(gpu, kind, c, n, hw, o, ks, stride):
+    """Tap-uniform convs of few output tiles (each wave of a workgroup walks every KW-th K tile, across filter
+    taps), with residual and ReLU, against the register-staged kernel (same bound as the GEMMs)."""
+    from hackathon_amd import _lib
+    from hackathon_amd.c35 import engine as E
+    from hackathon_amd.device import DeviceArray
+
+    rng = np.random.default_rng(n + hw + o + c)
+    pad, to = ks // 2, (lambda x: x) if kind == "fp32" else (lambda x: _bits(x, kind)[0])
+    ho = (hw + 2 * pad - ks) // stride + 1
+    x, w = rng.standard_normal((n, hw, hw, c), dtype=np.float32), rng.standard_normal((o, ks, ks, c), dtype=np.float32)
+    xd, wd, rd = _dev(to(x)), _dev(to(w)), _dev(to(rng.standard_normal((n, ho, ho, o), dtype=np.float32)))
+    bias = _dev(rng.standard_normal(o, dtype=np.float32))
+
+    def run():
+        out = DeviceArray.empty((n, ho, ho, o), xd.dtype)
+        a = _lib.ConvArgs()
+        a.x, a.w, a.out = xd.ptr, wd.ptr, out.ptr
+        a.n, a.c, a.h, a.w_, a.c_stride, a.c_pack, a.o, a.kh, a.kw, a.sh, a.sw = n, c, hw, hw, c, c, o, ks, ks, stride, stride
+        a.pad_top, a.pad_left, a.dh, a.dw, a.ho, a.wo = pad, pad, 1, 1, ho, ho
+        a.out_layout, a.in_dtype, a.out_dtype = 1, xd.code, xd.code
+        a.epi = E.epilogue(bias=bias, bias_mode=2, act=1, residual=rd)
+        _lib.launch(a)
+        return out.get()
+
+    got, want = run(), switches.with_switch("C3H_DISABLE_DMA", "1", run)
+    got, want = ((x if kind == "fp32" else _from16(x, kind)).astype(np.float64) for x in (got, want))
+    k = ks * ks * c  # |a b| sums to about 0.64 k on standard normals; 2 k bounds it
+    ulp = {"fp32": 2.0 ** -22, "bf16": 2.0 ** -7, "fp16": 2.0 ** -10}[kind]
+    assert np.all(np.abs(got - want) <= 2 * k * k * 2.0 ** -23 + ulp * np.abs(want)) and want.any()
