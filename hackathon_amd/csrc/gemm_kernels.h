@@ -2568,6 +2568,41 @@ int launch_ks_i8(Problem p, hipStream_t s, int mode, int out_dtype, int tile);  
 int launch_ks_f8(Problem p, hipStream_t s, int out_dtype, int tile);                 // gemm_ks_8.hip
 int launch_ks_f32(Problem p, hipStream_t s, int am, int tile);                       // gemm_ks_8.hip
 
+// Whether the four-wave DMA kernel takes this GEMM or conv on a 64-column
+// tile (0 = no, 1 = 64 x 64, 2 = 128 x 64): outputs whose 128 x 128 tiles
+// leave CUs idle or alone with one block, whose DMA wait, LDS reads and MFMAs
+// then follow one another unhidden (0.7 us per K tile at any stage count).
+// 64 x 64 up to two tiles per CU, 128 x 64 up to one 128 x 128 tile per CU --
+// and, for dense GEMMs of at most 1 KB of K per row, whose blocks are mostly
+// prologue and epilogue, up to 1.5.  Measured (bf16, M x N x K, us, 128 x 128
+// / 64 x 64 / 128 x 64): 700 x 2048 x 512 13.2 / 7.3 / 8.9, 3000 x 512 x 2048
+// 28.2 / 19.7 / 23.2, 8192 x 512 x 2048 27.8 / 28.8 / 24.9, 3000 x 2048 x 512
+// (384 tiles of 128 x 128) 18.2 / 16.6 / 13.7, 16384 x 512 x 512 (512) 14.6 /
+// 24.1 / 19.5; 3x3 convs of 128 channels 28 x 28: batch 20 16.1 / 11.4 /
+// 12.3, 37 (227 tiles) 16.9 / 16.5 / 14.5, 64 (392) 20.8 / 26.1 / 29.4.  The
+// K order is that of the other tiles: bit-identical results.
+inline int mid_tile(const Problem& p, int64_t batch, int cus, int am, int elem_bytes) {
+  if (!dma_eligible(p, batch, am)) return 0;
+  if (ceil_div(p.m, 64) * ceil_div(p.n, 64) <= 2 * cus) return 1;
+  const int64_t tiles128 = ceil_div(p.m, 128) * ceil_div(p.n, 128);
+  return tiles128 <= cus || (am == kDenseK && p.k * elem_bytes <= 1024 && 2 * tiles128 <= 3 * cus) ? 2 : 0;
+}
+template <typename Mma, typename TO, int AM>
+int launch_mid_tile(Problem p, hipStream_t s, int tile, const char* what) {
+  dim3 grid;
+  if (tile == 1) {
+    grid_of<64, 64>(p, 1, grid);
+    hipLaunchKernelGGL((mfma_gemm_dma_kernel<Mma, TO, 64, 64, 4, 1, AM, 2>), grid, dim3(kThreads), 0, s, p);
+  } else {
+    grid_of<128, 64>(p, 1, grid);
+    hipLaunchKernelGGL((mfma_gemm_dma_kernel<Mma, TO, 128, 64, 4, 1, AM, 2>), grid, dim3(kThreads), 0, s, p);
+  }
+  return launch_status(what);
+}
+int launch_mid_16(Problem p, hipStream_t s, int in_dtype, int am, int tile);         // gemm_mid_16.hip
+int launch_mid_i8(Problem p, hipStream_t s, int mode, int out_dtype, int tile);      // gemm_mid_8.hip
+int launch_mid_f8(Problem p, hipStream_t s, int out_dtype, int tile);                // gemm_mid_8.hip
+
 template <typename Mma, typename TO, int AM>
 int launch_mfma(Problem p, int64_t batch, hipStream_t s, const char* what) {
   dim3 grid;
@@ -2659,8 +2694,14 @@ int launch_mfma(Problem p, int64_t batch, hipStream_t s, const char* what) {
 template <typename Mma, typename T, int AM>
 int launch_h(Problem p, int64_t batch, hipStream_t s, int in_dtype) {
   if constexpr (AM == kDenseK || AM == kConvTap) {
-    if (p.out_dtype == C3H_F32 || p.out_dtype == in_dtype)
-      if (const int tile = ks_tile(p, batch, device_cus())) return launch_ks_16(p, s, in_dtype, AM, tile);
+    if (p.out_dtype == C3H_F32 || p.out_dtype == in_dtype) {
+      const int cus = device_cus();
+      // (Convs of at most 64 outputs keep the K-ordered kernel: the 64-channel
+      // band kernel is bit-identical to it at every size.)
+      const int ks = AM == kConvTap && p.n <= 64 ? 0 : ks_tile(p, batch, cus);
+      if (ks) return launch_ks_16(p, s, in_dtype, AM, ks);
+      if (const int tile = mid_tile(p, batch, cus, AM, 2)) return launch_mid_16(p, s, in_dtype, AM, tile);
+    }
   }
   if (p.out_dtype == C3H_F32) return launch_mfma<Mma, float, AM>(p, batch, s, "gemm_h");
   if (p.out_dtype == in_dtype) return launch_mfma<Mma, T, AM>(p, batch, s, "gemm_h");
@@ -2677,7 +2718,9 @@ int launch_h_any(Problem p, int64_t batch, hipStream_t s, int in_dtype) {
 // else the register-prefetch kernel.
 template <typename TO>
 int launch_fp8(Problem p, hipStream_t s) {
-  if (const int tile = ks_tile(p, 1, device_cus())) return launch_ks_f8(p, s, p.out_dtype, tile);
+  const int cus = device_cus();
+  if (const int tile = ks_tile(p, 1, cus)) return launch_ks_f8(p, s, p.out_dtype, tile);
+  if (const int tile = mid_tile(p, 1, cus, kDenseK, 1)) return launch_mid_f8(p, s, p.out_dtype, tile);
   dim3 grid;
   if (dma_eligible(p, 1, kDenseK) && big_tile_wins(p, device_cus(), sizeof(TO), false)) {
     grid_of<256, 256>(p, 1, grid);
