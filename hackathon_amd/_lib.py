@@ -34,7 +34,7 @@ OP_NOP, OP_EVENT_RECORD, OP_EVENT_WAIT, OP_COPY = 0, 1, 2, 3
 OP_FILL, OP_CAST, OP_EW, OP_STRIDED_COPY, OP_REDUCE, OP_SOFTMAX, OP_LAYERNORM, OP_BATCHNORM, \
     OP_GATHER, OP_ARGMAX, OP_IM2COL, OP_LAYOUT, OP_MAXPOOL, OP_GEMM, OP_CONV, OP_ATTN_SCORES, \
     OP_FLASH, OP_QUANTIZE, OP_QGEMM, OP_DEQUANTIZE, OP_BNFOLD, OP_PACK, OP_CONV_POOL, OP_QUANT_FP8, \
-    OP_GEMM_FP8, OP_SPLITK, OP_QUANT_MXFP4, OP_GEMM_W4A16, OP_ARGMAX_FINISH, OP_NONFINITE = range(10, 40)
+    OP_GEMM_FP8, OP_SPLITK, OP_QUANT_MXFP4, OP_GEMM_W4A16, OP_ARGMAX_FINISH, OP_NONFINITE, OP_FLASH_F32 = range(10, 41)
 
 vp = C.c_void_p
 i32 = C.c_int32
@@ -174,6 +174,10 @@ class FlashArgs(C.Structure):
                            "o_sb", "o_sh", "o_ss", "mask_ld")] + [("scale", f32), ("mask_kind", i32)]
 
 
+class FlashF32Args(FlashArgs):
+    """c3h_flash_args of the fp32 entry point."""
+
+
 class QuantizeArgs(C.Structure):
     _fields_ = [("x", vp), ("out", vp), ("count", i64), ("scale", f32), ("zero_point", i32),
                 ("x_dtype", i32), ("pad_", i32)]
@@ -248,7 +252,7 @@ KERNELS = {
     "c3h_batchnorm": BatchNormArgs, "c3h_bn_fold": BnFoldArgs, "c3h_gather": GatherArgs,
     "c3h_argmax": ArgmaxArgs, "c3h_im2col": Im2colArgs, "c3h_layout": LayoutArgs,
     "c3h_maxpool2d": PoolArgs, "c3h_gemm": GemmArgs, "c3h_conv2d": ConvArgs,
-    "c3h_attention_scores": AttnScoresArgs, "c3h_flash_attention": FlashArgs,
+    "c3h_attention_scores": AttnScoresArgs, "c3h_flash_attention": FlashArgs, "c3h_flash_attention_f32": FlashF32Args,
     "c3h_quantize": QuantizeArgs, "c3h_qgemm": QGemmArgs, "c3h_dequantize": DequantizeArgs,
     "c3h_pack_conv_weight": PackArgs, "c3h_conv_stem_pool": ConvPoolArgs,
     "c3h_quantize_fp8_rows": Fp8QuantArgs, "c3h_gemm_fp8": Fp8GemmArgs,
@@ -266,7 +270,7 @@ OP_KIND = {
     BnFoldArgs: OP_BNFOLD, PackArgs: OP_PACK, ConvPoolArgs: OP_CONV_POOL,
     Fp8QuantArgs: OP_QUANT_FP8, Fp8GemmArgs: OP_GEMM_FP8, SplitKArgs: OP_SPLITK,
     Mxfp4QuantArgs: OP_QUANT_MXFP4, W4A16GemmArgs: OP_GEMM_W4A16, ArgmaxFinishArgs: OP_ARGMAX_FINISH,
-    NonfiniteArgs: OP_NONFINITE,
+    NonfiniteArgs: OP_NONFINITE, FlashF32Args: OP_FLASH_F32,
 }
 
 KERNEL_OF_ARGS = {v: k for k, v in KERNELS.items()}

@@ -1648,7 +1648,7 @@ class CompiledPlan:
         div = self._scalar_const(node.inputs[2])
         pv = self._single_consumer(node.outputs[0])
         ok = (pv is not None and pv.op_type == "MatMul" and pv.inputs[0] == node.outputs[0]
-              and self.mm_code != _lib.F32 and q.shape[-1] == 64 and div is not None and div != 0.0
+              and q.shape[-1] == 64 and div is not None and div != 0.0
               and len(q.shape) == 4 and len(kt.shape) == 4 and q.shape[:2] == kt.shape[:2])
         mask = self._flash_mask(node.inputs[3], q.shape[2], kt.shape[3]) if ok else None
         if mask is None:
@@ -1672,7 +1672,7 @@ class CompiledPlan:
         ov = Val((b, h, s_q, d), dt, store.buf, 0, (s_q * h * d, d, h * d, 1))
 
         def build(r, qv=qv, kv=kv, vv=vv, store=store, mask_val=mask_val):
-            a = _lib.FlashArgs()
+            a = _lib.FlashF32Args() if dt == np.float32 else _lib.FlashArgs()
             a.q, a.k, a.v = self._ptr(qv, r), self._ptr(kv, r), self._ptr(vv, r)
             a.mask = self._ptr(mask_val, r) if mask_val is not None else None
             a.out = self._ptr(store, r)

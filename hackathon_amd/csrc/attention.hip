@@ -14,6 +14,8 @@
 //   the online-softmax state is then per lane and P^T feeds the O^T = V^T P^T
 //   MFMA straight from registers (both operands use the same key order, so
 //   the product is unchanged).
+//
+// flash_attention_f32: the same grouping for fp32 tensors, on the fp32 MFMA.
 #include "common.h"
 
 using namespace c3h;
@@ -410,9 +412,183 @@ __global__ void __launch_bounds__(256) flash_kernel(c3h_flash_args a) {
   }
 }
 
+// ------------------------------------------------------------ flash attention, fp32
+// The fp32 form: a workgroup owns 64 queries of one (batch, head), 16 per
+// wave, and walks 64-key tiles of K and V through LDS.  v_mfma_f32_16x16x4_f32
+// computes S^T = K Q^T, so a lane holds keys 4 g .. 4 g + 3 (+ 16 per tile
+// row) of its query; taking PV's K steps as keys {e, 4 + e, 8 + e, 12 + e}
+// makes those accumulators the P^T operand as they are.  All state is fp32
+// and p = exp(s - max) is the library's expf, as in the materialized form.
+//
+// Why: the materialized path (strided copies of Q, K^T, V and the context, a
+// VALU scores kernel that reads K^T column-strided, and a batched GEMM) was
+// bound by launches and by the scores kernel, which ran at 1 % of the MFMA
+// rate: 8 x 8 heads x 256 queries, 207 us of scores, 17 us of P V and 31 us of
+// copies per layer.  The MFMAs of this kernel are 8 us there.
+//
+// LDS rows are 68 floats (64 + 4): a lane group's K chunks and V rows then
+// fall on different banks.
+constexpr int kF32Row = kD + 4;
+
+template <int MASK>
+__global__ void __launch_bounds__(256) flash_f32_kernel(c3h_flash_args a) {
+  __shared__ __attribute__((aligned(16))) float Ks[kBK * kF32Row];
+  __shared__ __attribute__((aligned(16))) float Vs[kBK * kF32Row];
+  // Longest query tiles first, as in flash_kernel.
+  const int qtiles = (a.seq_q + 63) / 64;
+  const int nbh = a.batch * a.heads;
+  const int qt = qtiles - 1 - static_cast<int>(blockIdx.x / nbh);
+  const int bh = blockIdx.x % nbh;
+  const int head = bh % a.heads, batch = bh / a.heads;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int l16 = lane & 15, g = lane >> 4;
+  const float* Q = static_cast<const float*>(a.q) + batch * a.q_sb + head * a.q_sh;
+  const float* K = static_cast<const float*>(a.k) + batch * a.k_sb + head * a.k_sh;
+  const float* V = static_cast<const float*>(a.v) + batch * a.v_sb + head * a.v_sh;
+  float* O = static_cast<float*>(a.out) + batch * a.o_sb + head * a.o_sh;
+  const float* mask = static_cast<const float*>(a.mask);
+
+  const int wave_q1 = qt * 64 + wave * 16 + 15;  // this wave's last query
+  const int q = qt * 64 + wave * 16 + l16;       // this lane's
+  const bool q_valid = q < a.seq_q;
+  f32x4 qf[4];  // dims 16 c + 4 g .. + 3
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    qf[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (q_valid) qf[c] = *reinterpret_cast<const f32x4*>(Q + q * a.q_ss + 16 * c + 4 * g);
+  }
+  f32x4 o[4];  // O^T: dims 16 d + 4 g + r
+#pragma unroll
+  for (int d = 0; d < 4; ++d) o[d] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m = -INFINITY, l = 0.0f;  // running maximum of the query; this lane's share of the sum
+
+  const int kend = MASK == 1 ? min(a.seq_k, qt * 64 + 64) : a.seq_k;
+  const int ntiles = (kend + kBK - 1) / kBK;
+  // Staging: four 16-byte loads of K and of V per thread, the four threads of
+  // a row on 64 consecutive bytes; keys past seq_k read zeros.
+  const int row = tid >> 2, dim = (tid & 3) * 4;
+  f32x4 kreg[4], vreg[4];
+  auto load_tile = [&](int t) {
+    const int key = t * kBK + row;
+    const bool ok = key < a.seq_k;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      kreg[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+      vreg[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (ok) {
+        kreg[i] = *reinterpret_cast<const f32x4*>(K + key * a.k_ss + dim + 16 * i);
+        vreg[i] = *reinterpret_cast<const f32x4*>(V + key * a.v_ss + dim + 16 * i);
+      }
+    }
+  };
+  if (ntiles > 0) load_tile(0);
+  for (int t = 0; t < ntiles; ++t) {
+    const int k0 = t * kBK;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      *reinterpret_cast<f32x4*>(Ks + row * kF32Row + dim + 16 * i) = kreg[i];
+      *reinterpret_cast<f32x4*>(Vs + row * kF32Row + dim + 16 * i) = vreg[i];
+    }
+    __syncthreads();
+    if (t + 1 < ntiles) load_tile(t + 1);  // in flight while this tile is multiplied
+    // Causal: a tile wholly after this wave's last query contributes nothing.
+    if (MASK != 1 || k0 <= wave_q1) {
+      f32x4 s[4];  // keys k0 + 16 j + 4 g + r
+#pragma unroll
+      for (int j = 0; j < 4; ++j) s[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        f32x4 kf[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          kf[j] = *reinterpret_cast<const f32x4*>(Ks + (16 * j + l16) * kF32Row + 16 * c + 4 * g);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) s[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[j][e], qf[c][e], s[j], 0, 0, 0);
+      }
+      float tmax = -INFINITY;
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int key = k0 + 16 * j + 4 * g + r;
+          float v = s[j][r] * a.scale;
+          if (MASK == 2 && q_valid && key < a.seq_k) v += mask[static_cast<int64_t>(q) * a.mask_ld + key];
+          if (key >= a.seq_k || (MASK == 1 && key > q)) v = -INFINITY;
+          s[j][r] = v;
+          tmax = fmaxf(tmax, v);
+        }
+      tmax = fmaxf(tmax, __shfl_xor(tmax, 16, 64));
+      tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
+      const float m_new = fmaxf(m, tmax);
+      // A row with no finite score yet keeps p = 0 (exp(-inf)); one that
+      // never gets one ends as 0 / 0, the materialized softmax's NaN.
+      const float base = m_new == -INFINITY ? 0.0f : m_new;
+      const float corr = m == -INFINITY ? 0.0f : expf(m - base);
+      m = m_new;
+      l *= corr;
+#pragma unroll
+      for (int d = 0; d < 4; ++d) o[d] *= corr;
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          s[j][r] = expf(s[j][r] - base);
+          l += s[j][r];
+        }
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float* vrow = Vs + (16 * j + 4 * g + e) * kF32Row + l16;
+#pragma unroll
+          for (int d = 0; d < 4; ++d)
+            o[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(vrow[16 * d], s[j][e], o[d], 0, 0, 0);
+        }
+    }
+    __syncthreads();
+  }
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
+  if (q_valid) {
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+      f32x4 v;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] = o[d][r] / l;
+      *reinterpret_cast<f32x4*>(O + q * a.o_ss + 16 * d + 4 * g) = v;
+    }
+  }
+}
+
 }  // namespace
 
 extern "C" {
+
+int c3h_flash_attention_f32(const c3h_flash_args* a, void* stream) {
+  C3H_REQUIRE(a != nullptr, "flash_f32: null args");
+  C3H_REQUIRE(a->dtype == C3H_F32, "flash_f32: dtype must be fp32");
+  C3H_REQUIRE(a->head_dim == kD, "flash_f32: head_dim %d unsupported (needs 64)", a->head_dim);
+  C3H_REQUIRE(a->batch >= 0 && a->heads >= 1 && a->seq_q >= 0 && a->seq_k >= 1, "flash_f32: bad sizes");
+  C3H_REQUIRE(a->mask_kind >= 0 && a->mask_kind <= 2, "flash_f32: bad mask_kind");
+  C3H_REQUIRE(a->mask_kind != 2 || a->mask != nullptr, "flash_f32: additive mask pointer missing");
+  C3H_REQUIRE(((a->q_sb | a->q_sh | a->q_ss | a->k_sb | a->k_sh | a->k_ss | a->v_sb | a->v_sh | a->v_ss | a->o_sb |
+                a->o_sh | a->o_ss) & 3) == 0,
+              "flash_f32: strides must be multiples of 4 elements");
+  C3H_REQUIRE(((reinterpret_cast<uintptr_t>(a->q) | reinterpret_cast<uintptr_t>(a->k) |
+                reinterpret_cast<uintptr_t>(a->v) | reinterpret_cast<uintptr_t>(a->out)) & 15) == 0,
+              "flash_f32: misaligned operands");
+  if (a->batch == 0 || a->seq_q == 0) return C3H_OK;
+  const int64_t blocks = static_cast<int64_t>(a->batch) * a->heads * ((a->seq_q + 63) / 64);
+  C3H_REQUIRE(blocks <= 2147483647LL, "flash_f32: too many workgroups");
+  const dim3 grid(static_cast<unsigned>(blocks));
+  hipStream_t s = as_stream(stream);
+  if (a->mask_kind == 0) hipLaunchKernelGGL(flash_f32_kernel<0>, grid, dim3(256), 0, s, *a);
+  else if (a->mask_kind == 1) hipLaunchKernelGGL(flash_f32_kernel<1>, grid, dim3(256), 0, s, *a);
+  else hipLaunchKernelGGL(flash_f32_kernel<2>, grid, dim3(256), 0, s, *a);
+  return launch_status("flash_attention_f32");
+}
 
 int c3h_attention_scores(const c3h_attn_scores_args* a, void* stream) {
   C3H_REQUIRE(a != nullptr, "attention_scores: null args");

@@ -307,6 +307,7 @@ static int dispatch_op(const c3h_op& op, hipStream_t s, void* const* events, int
     case C3H_OP_GEMM: return c3h_gemm(static_cast<const c3h_gemm_args*>(op.args), s);
     case C3H_OP_CONV: return c3h_conv2d(static_cast<const c3h_conv_args*>(op.args), s);
     case C3H_OP_ATTN_SCORES: return c3h_attention_scores(static_cast<const c3h_attn_scores_args*>(op.args), s);
+    case C3H_OP_FLASH_F32: return c3h_flash_attention_f32(static_cast<const c3h_flash_args*>(op.args), s);
     case C3H_OP_FLASH: return c3h_flash_attention(static_cast<const c3h_flash_args*>(op.args), s);
     case C3H_OP_QUANTIZE: return c3h_quantize(static_cast<const c3h_quantize_args*>(op.args), s);
     case C3H_OP_QGEMM: return c3h_qgemm(static_cast<const c3h_qgemm_args*>(op.args), s);

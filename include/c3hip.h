@@ -616,6 +616,11 @@ typedef struct {
   int32_t mask_kind;
 } c3h_flash_args;
 int c3h_flash_attention(const c3h_flash_args* a, void* stream);
+/* The same for dtype F32 tensors (strides multiples of 4 elements, 16-byte
+ * aligned, no extent limit), in fp32 throughout: exp(s - max) with the
+ * library's expf, P and its sum in fp32.  `scale` may have any sign.  A row
+ * whose every score is -inf gives NaN, as the materialized softmax does. */
+int c3h_flash_attention_f32(const c3h_flash_args* a, void* stream);
 
 /* ------------------------------------------------------------------ */
 /* W8A8 (QuantizeLinear / QLinearMatMul / DequantizeLinear)             */
@@ -854,7 +859,8 @@ enum c3h_op_kind {
   C3H_OP_QUANT_MXFP4 = 36,
   C3H_OP_GEMM_W4A16 = 37,
   C3H_OP_ARGMAX_FINISH = 38,
-  C3H_OP_NONFINITE = 39
+  C3H_OP_NONFINITE = 39,
+  C3H_OP_FLASH_F32 = 40
 };
 
 typedef struct {

@@ -1770,3 +1770,47 @@ def test_small_output_conv_matches_the_general_kernel(gpu, kind, c, n, hw, o, ks
     k = ks * ks * c  # |a b| sums to about 0.64 k on standard normals; 2 k bounds it
     ulp = {"fp32": 2.0 ** -22, "bf16": 2.0 ** -7, "fp16": 2.0 ** -10}[kind]
     assert np.all(np.abs(got - want) <= 2 * k * k * 2.0 ** -23 + ulp * np.abs(want)) and want.any()
+
+
+@pytest.mark.parametrize("mask_kind", [0, 1, 2])
+@pytest.mark.parametrize("b,h,sq,sk", [(1, 1, 1, 1), (2, 3, 18, 18), (1, 2, 64, 65), (1, 2, 129, 200), (3, 1, 63, 257)])
+def test_flash_attention_fp32(gpu, b, h, sq, sk, mask_kind):
+    """fp32 flash attention on packed QKV views: one query, ragged query and key tiles, each mask kind (an
+    additive row of -inf gives NaN, as the materialized softmax does), against float64.  A score is within
+    72 2^-24 of its sum |q k| / 8, which moves each weight by that share (twice: numerator and sum), and the
+    weighted sum of S keys adds (S + 8) 2^-24."""
+    from hackathon_amd import _lib
+    from hackathon_amd.device import DeviceArray
+
+    if mask_kind == 1:
+        sk = sq
+    rng = np.random.default_rng(sq + sk + mask_kind)
+    w, s = 3 * h * 64, max(sq, sk)
+    qkv = rng.standard_normal((b, s, w), dtype=np.float32)
+    mask = (rng.standard_normal((sq, sk)) * 2).astype(np.float32)
+    mask[rng.random((sq, sk)) < 0.2] = -np.inf
+    mask[sq // 2] = -np.inf
+    d, md, out = _dev(qkv), _dev(mask), DeviceArray.empty((b, sq, h, 64), np.float32)
+    a = _lib.FlashF32Args()
+    a.q, a.k, a.v, a.mask, a.out = d.ptr, d.ptr + 4 * 64 * h, d.ptr + 8 * 64 * h, md.ptr, out.ptr
+    a.batch, a.heads, a.seq_q, a.seq_k, a.head_dim, a.dtype = b, h, sq, sk, 64, _lib.F32
+    for t in "qkv":
+        setattr(a, t + "_sb", s * w), setattr(a, t + "_sh", 64), setattr(a, t + "_ss", w)
+    a.o_sb, a.o_sh, a.o_ss, a.mask_ld, a.scale, a.mask_kind = sq * h * 64, 64, h * 64, sk, 0.125, mask_kind
+    _lib.launch(a)
+    q, k, v = (x.reshape(b, s, h, 64).transpose(0, 2, 1, 3).astype(np.float64) for x in np.split(qkv, 3, axis=-1))
+    q, k, v = q[:, :, :sq], k[:, :, :sk], v[:, :, :sk]
+    sc = q @ k.transpose(0, 1, 3, 2) / 8
+    size = np.max(np.abs(q) @ np.abs(k).transpose(0, 1, 3, 2) / 8 + np.where(mask_kind == 2, 8, 0))
+    if mask_kind == 1:
+        sc = np.where(np.triu(np.ones((sq, sk), bool), 1), -np.inf, sc)
+    elif mask_kind == 2:
+        sc = sc + mask
+    with np.errstate(invalid="ignore"):
+        p = np.exp(sc - sc.max(-1, keepdims=True))
+        ref = (p / p.sum(-1, keepdims=True)) @ v
+    got = out.get().transpose(0, 2, 1, 3)
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(ref))
+    assert mask_kind != 2 or np.isnan(got[:, :, sq // 2]).all()
+    bound = (2 * 72 * size + sk + 8) * 2.0 ** -24 * np.max(np.abs(v))
+    assert np.nanmax(np.abs(got - ref), initial=0.0) <= bound
