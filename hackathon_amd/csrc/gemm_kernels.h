@@ -2744,18 +2744,27 @@ int launch_fp8(Problem p, hipStream_t s) {
 }
 
 // W4A16 GEMM: the register-prefetch kernel with MXFP4 B and buffer loads.
+template <typename TO, int BM, int BN, int WM, int WN>
+int launch_w4_tile(Problem p, hipStream_t s) {
+  dim3 grid;
+  grid_of<BM, BN>(p, 1, grid);
+  hipLaunchKernelGGL((mfma_gemm_kernel<MmaF16, TO, BM, BN, WM, WN, kDenseK, true, true>), grid, dim3(kThreads), 0, s, p);
+  return launch_status("gemm_w4a16");
+}
+// 64 x 64 tiles up to four per CU, then 128 x 64 up to 1.5 tiles of 128 x 128
+// per CU, or past two where K is at most 1024 (the epilogue's share is large);
+// measured (M x N x K, us, 128 x 128 / 64 x 64 / 128 x 64): 200 x 512 x 2048
+// 34.4 / 17.4 / 23.5, 3000 x 512 x 2048 37.6 / 24.4 / 26.9, 3000 x 2048 x 512
+// 22.8 / 20.3 / 18.7, 6000 x 768 x 3072 63.1 / 66.5 / 55.2, 6000 x 2304 x 768
+// 48.3 / 49.0 / 44.9, 16384 x 512 x 2048 49.9 / 64.2 / 58.6.  Every tile sums
+// K in the same order.
 template <typename TO>
 int launch_w4(Problem p, hipStream_t s) {
-  dim3 grid;
-  if (p.n <= 64) {
-    grid_of<256, 64>(p, 1, grid);
-    hipLaunchKernelGGL((mfma_gemm_kernel<MmaF16, TO, 256, 64, 4, 1, kDenseK, true, true>), grid, dim3(kThreads), 0, s, p);
-  } else {
-    grid_of<128, 128>(p, 1, grid);
-    hipLaunchKernelGGL((mfma_gemm_kernel<MmaF16, TO, 128, 128, 2, 2, kDenseK, true, true>), grid, dim3(kThreads), 0, s,
-                       p);
-  }
-  return launch_status("gemm_w4a16");
+  const int64_t cus = device_cus(), tiles128 = ceil_div(p.m, 128) * ceil_div(p.n, 128);
+  if (ceil_div(p.m, 64) * ceil_div(p.n, 64) <= 4 * cus) return launch_w4_tile<TO, 64, 64, 4, 1>(p, s);
+  if (p.n <= 64) return launch_w4_tile<TO, 256, 64, 4, 1>(p, s);
+  if (2 * tiles128 <= 3 * cus || (p.k <= 1024 && tiles128 > 2 * cus)) return launch_w4_tile<TO, 128, 64, 4, 1>(p, s);
+  return launch_w4_tile<TO, 128, 128, 2, 2>(p, s);
 }
 
 // row_max_ok: the entry point can compute the row_max side output (it is

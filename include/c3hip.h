@@ -802,7 +802,9 @@ int c3h_quantize_mxfp4(const c3h_mxfp4_quant_args* a, void* stream);
  * W[n,k] = E2M1(codes) * 2^(scales[n][k/32] - 127) widened to fp16 in
  * registers (exact under c3h_quantize_mxfp4's exponent range), fp16 MFMA
  * with fp32 accumulation, and the common epilogue into fp32 or fp16.
- * Equals c3h_gemm on the dequantized fp16 weights bit for bit.  k % 32 == 0,
+ * Equals, bit for bit, the fp16 GEMM of the dequantized weights that sums K
+ * in order (c3h_gemm's result, except where it splits the K of an output of
+ * few tiles over the waves of a workgroup).  k % 32 == 0,
  * lda % 8 == 0, ldb (bytes) % 4 == 0 and >= k/2, ldbs >= k/32; A 16-byte
  * aligned; A, codes and scales each below 2^31 bytes. */
 typedef struct {

@@ -204,3 +204,17 @@ def test_gemm_w4a16_host_checks(gpu):
     q.x, q.codes, q.scales, q.rows, q.cols, q.ldx, q.ldc, q.lds, q.x_dtype = a.ptr, c.ptr, s.ptr, 32, 48, 64, 32, 2, _lib.F16
     with pytest.raises(_lib.C3HError, match="multiple of 32"):
         _lib.launch(q, None)
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 10, 32), (65, 67, 96), (2100, 2050, 64), (2050, 3000, 1056), (70000, 40, 32)])
+def test_gemm_w4a16_tiles_sum_k_in_one_order(gpu, m, n, k):
+    """The 64 x 64, 128 x 64, 128 x 128 and 256 x 64 tiles at ragged edges: bit-identical to the K-ordered fp16
+    GEMM of the dequantized weights."""
+    rng = np.random.default_rng(m + n + k)
+    a16 = rng.standard_normal((m, k), dtype=np.float32).astype(np.float16)
+    codes = rng.integers(0, 256, (n, k // 2)).astype(np.uint8)
+    scales = rng.integers(120, 130, (n, k // 32)).astype(np.uint8)
+    w16 = F4.dequantize_mxfp4(codes, scales).astype(np.float16)
+    got = _w4_gpu(a16, codes, scales, n, k)
+    want = switches.with_switch("C3H_DISABLE_DMA", "1", lambda: _f16_gpu(a16, w16))
+    np.testing.assert_array_equal(got.view(np.uint8), want.view(np.uint8))
