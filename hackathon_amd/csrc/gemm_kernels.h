@@ -2356,7 +2356,13 @@ __global__ void __launch_bounds__(NW * 64) mfma_gemm_dma_kernel(Problem p) {
     // other waits on its DMA, barrier and LDS reads.
     if constexpr (kPrio) __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-    for (int q = 0; q < KS; ++q) mma_step<Mma, TM, TN>(acc, av[q], bv[q]);
+    for (int q = 0; q < KS; ++q)
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          acc[i][j] = Mma::mma(bv[q][j], av[q][i], acc[i][j]);  // C^T: see epilogue_direct
+        }
     if constexpr (kPrio) __builtin_amdgcn_s_setprio(0);
     __builtin_amdgcn_sched_barrier(0);
   }
