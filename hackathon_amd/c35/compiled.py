@@ -59,6 +59,7 @@ _MM_CODE = {"fp32": _lib.F32, "bf16": _lib.BF16, "fp16": _lib.F16, "w8a8": _lib.
 # c3h_layernorm's vector path (the only one with an int8 output): 8-wide
 # vectors, at most 8 per lane of one wave (memory_bound.hip: 512 * kLnVec).
 LN_QUANT_MAX_COLS = 4096
+DIRECT_LAUNCHES = 4  # programs this short skip the graph replay
 
 
 def quant_scale_ok(scale: float) -> bool:
@@ -574,8 +575,11 @@ class CompiledPlan:
                 self._stream.synchronize()
 
     def launch(self) -> None:
-        """Enqueue the whole program (hipGraph replay when captured)."""
-        if self._graph_exec is not None:
+        """Enqueue the whole program: as a hipGraph replay when captured, but
+        launch by launch when it has at most `DIRECT_LAUNCHES` of them (a replay
+        costs about as much as three launches: the MLP, launch to finish, 32 us
+        replayed and 27 us direct)."""
+        if self._graph_exec is not None and len(self.launches) > DIRECT_LAUNCHES:
             _lib.check(_lib.lib().c3h_graph_launch(self._graph_exec, self._stream.handle), "c3h_graph_launch")
         else:
             _lib.check(_lib.lib().c3h_program_run(self._prog, self._n_prog, self._prog_streams,
@@ -1570,11 +1574,23 @@ class CompiledPlan:
             return None, None
         return add, self._weight_val(others[0], np.float32)
 
-    def _error_flag(self) -> DeviceArray:
-        """A device int32 that kernels set to 1 on an invalid index (sticky until read)."""
+    def _error_flag(self) -> PinnedArray:
+        """A pinned host int32 that kernels set to 1 on an invalid index (sticky
+        until read).  Only a bad index writes it, so it costs the kernels
+        nothing, and the host reads it without a copy: a device flag took a
+        device-wide synchronize and a 4-byte copy after every run (23 us of a
+        one-sequence decoder's 283)."""
         if getattr(self, "_errflag", None) is None:
-            self._errflag = self._keep(DeviceArray.from_host(np.zeros(1, np.int32)))
+            self._errflag = self._keep(PinnedArray((1,), np.int32))
+            a = _lib.FillArgs()  # by a kernel on the null stream: finished before the plan's stream runs
+            a.out, a.count, a.dtype, a.value = self._errflag.ptr, 1, _lib.I32, 0.0
+            _lib.launch(a, None)
         return self._errflag
+
+    @property
+    def error_flag(self) -> Optional[PinnedArray]:
+        """The pinned int32 that is nonzero after a bad index, or None when no launch checks one."""
+        return getattr(self, "_errflag", None)
 
     def read_value(self, name: str, rows: Optional[int] = None) -> np.ndarray:
         """Host copy of a value this program stores, in its logical (ONNX)
@@ -1609,14 +1625,14 @@ class CompiledPlan:
 
     def check_errors(self) -> None:
         """Raise IndexError if a kernel of this program saw an out-of-range
-        index since the last check (the flag is cleared after reading).  A
-        synchronous 4-byte read: call it after the program's stream has
-        finished, outside any timed region."""
-        flag = getattr(self, "_errflag", None)
+        index since the last check (the flag is cleared after reading).
+        Waits for the program's stream."""
+        flag = self.error_flag
         if flag is None:
             return
-        if int(flag.get()[0]) != 0:
-            flag.copy_from_host(np.zeros(1, np.int32))
+        self._stream.synchronize()
+        if int(flag.array[0]) != 0:
+            flag.array[0] = 0
             raise IndexError("Gather: an index is out of bounds for the gathered axis (ONNX Gather requires "
                              "-axis_dim <= index < axis_dim)")
 

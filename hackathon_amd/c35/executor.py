@@ -665,7 +665,6 @@ def _stream_compiled(pipeline, arrays, total, batch, out_name, out_path,
     ready = [Event(), Event()]
     chunks = [kept(("chunk", k), lambda: PinnedArray((_CHUNK_BYTES // 4,), np.float32)) for k in range(2)]
     chunk_done = [Event(), Event()]
-    flags = [PinnedArray((1,), np.int32) for _ in range(2)]  # each batch's gather error flag
     nf_dev = [DeviceArray.empty((1,), np.int32) for _ in range(2)]  # each batch's non-finite flag
     nf_host = [PinnedArray((1,), np.int32) for _ in range(2)]
     progs: list = [None, None]
@@ -678,8 +677,6 @@ def _stream_compiled(pipeline, arrays, total, batch, out_name, out_path,
 
     def drain(slot, start, end):
         copy_stream.wait_event(ready[slot])
-        flag = progs[slot]._error_flag()
-        _lib.check(_lib.lib().c3h_memcpy_d2h_async(flags[slot].ptr, flag.ptr, 4, copy_stream.handle), "d2h")
         _lib.check(_lib.lib().c3h_memcpy_d2h_async(nf_host[slot].ptr, nf_dev[slot].ptr, 4, copy_stream.handle), "d2h")
         src = stage[slot]
         row = math.prod(tail)
@@ -694,7 +691,8 @@ def _stream_compiled(pipeline, arrays, total, batch, out_name, out_path,
             chunk_done[k % 2].record(copy_stream)
 
         def check_flags():
-            if int(flags[slot].array[0]) != 0:
+            flag = progs[slot].error_flag
+            if flag is not None and int(flag.array[0]) != 0:
                 progs[slot].check_errors()  # clears the flag and raises IndexError
             if int(nf_host[slot].array[0]) != 0:
                 raise ValueError("Output contains non-finite values (NaN or Inf)")
@@ -707,7 +705,7 @@ def _stream_compiled(pipeline, arrays, total, batch, out_name, out_path,
         for k, (o0, o1) in enumerate(spans):
             if k + 1 < len(spans):
                 issue(k + 1)
-            chunk_done[k % 2].synchronize()  # the flag copies were queued before chunk 0
+            chunk_done[k % 2].synchronize()  # the batch is done, and its flag copy was queued before chunk 0
             if k == 0:
                 check_flags()
             mm.write(o0, chunks[k % 2].array[: o1 - o0])
