@@ -7,8 +7,8 @@
 //   recomputes each three times).
 //
 // flash_attention: the launch-grouped FusedAttentionScores + P.V MatMul.  A
-//   workgroup owns 128 queries of one (batch, head) (two groups of 16 per
-//   wave); K and V tiles of 64 keys are staged in LDS, the next tile's loads
+//   workgroup owns 128 or 64 queries of one (batch, head) (two groups of 16,
+//   or one, per wave); K and V tiles of 64 keys are staged in LDS, the next tile's loads
 //   in flight while the current one is multiplied.  Each wave computes S^T = K Q^T with
 //   v_mfma_f32_16x16x32_{f16,bf16} so that a lane holds one query's scores;
 //   the online-softmax state is then per lane and P^T feeds the O^T = V^T P^T
@@ -83,8 +83,6 @@ __global__ void __launch_bounds__(kScoreThreads) attention_scores_kernel(c3h_att
 
 // ------------------------------------------------------------ flash attention
 constexpr int kD = 64;        // head dim
-constexpr int QG = 2;         // 16-query groups per wave
-constexpr int kBQ = 64 * QG;  // queries per workgroup
 constexpr int kBK = 64;       // keys per tile
 constexpr float kLog2e = 1.4426950408889634f;
 // Lazy rescaling: the exponent base of a query moves to its running maximum
@@ -126,9 +124,10 @@ template <> __device__ __forceinline__ uint32_t pack2<f16_t>(float lo, float hi)
 
 // Each wave owns QG groups of 16 queries (kBQ = 64 * QG per workgroup): every
 // K / V^T fragment read from LDS feeds QG MFMAs, and the tile staging is
-// shared by 4 * 16 * QG queries.
-template <typename T, int MASK>
+// shared by 4 * 16 * QG queries.  A group's arithmetic does not depend on QG.
+template <typename T, int MASK, int QG>
 __global__ void __launch_bounds__(256) flash_kernel(c3h_flash_args a) {
+  constexpr int kBQ = 64 * QG;  // queries per workgroup
   typedef typename FlashMma<T>::vec vec8;
   __shared__ __attribute__((aligned(16))) uint8_t Ks[kBK * 128];
   __shared__ __attribute__((aligned(16))) uint8_t Vt[kD * 128];
@@ -631,15 +630,32 @@ int c3h_flash_attention(const c3h_flash_args* a, void* stream) {
                   (static_cast<int64_t>(a->seq_k - 1) * a->v_ss + kD) * 2 < (int64_t{1} << 31),
               "flash: one head's K or V spans 2 GiB or more");
   if (a->batch == 0 || a->seq_q == 0) return C3H_OK;
-  int64_t blocks = static_cast<int64_t>(a->batch) * a->heads * ((a->seq_q + kBQ - 1) / kBQ);
+  // 128 queries per workgroup (each K / V fragment feeds two MFMAs), or 64
+  // where 128 make at most two workgroups per CU -- the longest walk over the
+  // keys is then the kernel's length, and its tiles are half as long -- and
+  // for short causal sequences, whose 128-query tiles are half masked.
+  // Same bits.  us at 128 / 64 queries (batch x heads x sequence, causal):
+  // 1 x 8 x 200 8.5 / 6.3, 1 x 12 x 2048 44.5 / 33.2, 32 x 8 x 256 (512
+  // workgroups of 128) 11.0 / 9.8, 64 x 8 x 256 20.4 / 18.6, 100 x 8 x 128
+  // 15.8 / 12.4; 8 x 12 x 1000 (768) 29.9 / 32.1, 16 x 12 x 1024 49.3 / 53.1.
+  const int64_t bh = static_cast<int64_t>(a->batch) * a->heads;
+  int dev = 0, cus = 256;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+    cus = 256;
+  const bool half = bh * ((a->seq_q + 127) / 128) <= 2 * cus || (a->mask_kind == 1 && a->seq_q <= 256);
+  const int64_t blocks = bh * (half ? (a->seq_q + 63) / 64 : (a->seq_q + 127) / 128);
   C3H_REQUIRE(blocks <= 2147483647LL, "flash: too many workgroups");
   hipStream_t s = as_stream(stream);
   dim3 grid(static_cast<unsigned>(blocks));
-#define C3H_FLASH_LAUNCH(T)                                                                            \
-  switch (a->mask_kind) {                                                                              \
-    case 0: hipLaunchKernelGGL((flash_kernel<T, 0>), grid, dim3(256), 0, s, *a); break;                \
-    case 1: hipLaunchKernelGGL((flash_kernel<T, 1>), grid, dim3(256), 0, s, *a); break;                \
-    default: hipLaunchKernelGGL((flash_kernel<T, 2>), grid, dim3(256), 0, s, *a); break;               \
+#define C3H_FLASH_LAUNCH_QG(T, M)                                                              \
+  if (half) hipLaunchKernelGGL((flash_kernel<T, M, 1>), grid, dim3(256), 0, s, *a);            \
+  else hipLaunchKernelGGL((flash_kernel<T, M, 2>), grid, dim3(256), 0, s, *a)
+#define C3H_FLASH_LAUNCH(T)                                \
+  switch (a->mask_kind) {                                  \
+    case 0: C3H_FLASH_LAUNCH_QG(T, 0); break;              \
+    case 1: C3H_FLASH_LAUNCH_QG(T, 1); break;              \
+    default: C3H_FLASH_LAUNCH_QG(T, 2); break;             \
   }
   if (a->dtype == C3H_BF16) {
     C3H_FLASH_LAUNCH(bf16_t)
@@ -649,6 +665,7 @@ int c3h_flash_attention(const c3h_flash_args* a, void* stream) {
     return fail(C3H_EUNSUPPORTED, "flash: dtype %d unsupported", a->dtype);
   }
 #undef C3H_FLASH_LAUNCH
+#undef C3H_FLASH_LAUNCH_QG
   return launch_status("flash_attention");
 }
 

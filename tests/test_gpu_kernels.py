@@ -1682,7 +1682,7 @@ def test_conv_fp32_pipeline_edges(gpu, n, h, w, c, o, ks, stride, nchw):
 @pytest.mark.parametrize("kind", ["fp32", "fp16", "bf16", "fp8", "int8"])
 @pytest.mark.parametrize("m,n,k,ldo,form", [
     (1, 10, 64, 10, "relu"), (17, 33, 144, 40, "program"), (16, 32, 2048, 32, "gelu"),   # 16 x 32 tiles
-    (515, 289, 272, 292, "relu"), (1000, 512, 1040, 512, "gelu")])                      # 32 x 32 tiles
+    (515, 289, 272, 292, "relu"), (1000, 512, 1040, 512, "gelu"), (700, 770, 6144, 772, "program")])  # 32 x 32
 def test_small_output_gemm_matches_the_general_kernel(gpu, kind, m, n, k, ldo, form):
     """GEMMs of few output tiles split K over the waves of a workgroup: one row, ragged edges, fewer K tiles
     than waves, a partial last K tile and strided output rows, against the register-staged kernel
@@ -1814,3 +1814,33 @@ def test_flash_attention_fp32(gpu, b, h, sq, sk, mask_kind):
     assert mask_kind != 2 or np.isnan(got[:, :, sq // 2]).all()
     bound = (2 * 72 * size + sk + 8) * 2.0 ** -24 * np.max(np.abs(v))
     assert np.nanmax(np.abs(got - ref), initial=0.0) <= bound
+
+
+@pytest.mark.parametrize("kind", ["bf16", "fp16"])
+@pytest.mark.parametrize("s,mask_kind", [(260, 1), (130, 0), (129, 2)])
+def test_flash_attention_query_tiles_give_the_same_bits(gpu, kind, s, mask_kind):
+    """Workgroups of 64 queries (a batch of one) and of 128 (batches past two workgroups per CU): a query's
+    arithmetic is the same in both."""
+    from hackathon_amd import _lib
+    from hackathon_amd.device import DeviceArray
+
+    h, w = 8, 3 * 8 * 64
+    b = 2 * gpu.device_props().compute_units // (h * -(-s // 128)) + 2
+    rng = np.random.default_rng(s)
+    bits, _ = _bits(rng.standard_normal((b, s, w), dtype=np.float32), kind)
+    qkv, mask = _dev(bits), _dev((rng.standard_normal((s, s)) * 2).astype(np.float32))
+    both = DeviceArray.empty((b, s, h, 64), qkv.dtype), DeviceArray.empty((b, s, h, 64), qkv.dtype)
+    row_in, row_out = s * w * 2, s * h * 64 * 2
+    for out, batches in zip(both, ([(0, b)], [(i, 1) for i in (0, b // 2, b - 1)])):
+        for i, n in batches:
+            a = _lib.FlashArgs()
+            p = qkv.ptr + i * row_in
+            a.q, a.k, a.v, a.mask, a.out = p, p + 2 * 64 * h, p + 4 * 64 * h, mask.ptr, out.ptr + i * row_out
+            a.batch, a.heads, a.seq_q, a.seq_k, a.head_dim, a.dtype = n, h, s, s, 64, qkv.code
+            for t in "qkv":
+                setattr(a, t + "_sb", s * w), setattr(a, t + "_sh", 64), setattr(a, t + "_ss", w)
+            a.o_sb, a.o_sh, a.o_ss, a.mask_ld, a.scale, a.mask_kind = s * h * 64, 64, h * 64, s, 0.125, mask_kind
+            _lib.launch(a)
+    large, small = (x.get() for x in both)
+    for i in (0, b // 2, b - 1):
+        np.testing.assert_array_equal(large[i].view(np.uint16), small[i].view(np.uint16))
