@@ -77,7 +77,7 @@ int c3h_gemm(const c3h_gemm_args* a, void* stream) {
     bool b_ok = aligned(a->b, 16) && (a->ldb % 4 == 0) && (a->stride_b % 4 == 0);
     // Outputs too small for the 64 x 64 tiles, unless the small-output kernel
     // reads these operands (launch_f32_modes): 1 x 512 x 512 54 against 5 us.
-    const bool k_rows = !a->trans_a && a->trans_b && a->k % 4 == 0 && ks_tile(p, a->batch, device_cus()) != 0;
+    const bool k_rows = !a->trans_a && a->trans_b && a->k % 4 == 0 && ks_tile(p, a->batch, device_cus(), 4) != 0;
     if (!(a_ok && b_ok) || (a->m * a->n * a->batch < 4096 && !k_rows)) {
       dim3 grid(static_cast<unsigned>(ceil_div(a->n, 16)), static_cast<unsigned>(ceil_div(a->m, 16)),
                 static_cast<unsigned>(a->batch));

@@ -129,12 +129,13 @@ int launch_f32_dma(Problem p, hipStream_t s) {
 int launch_f32_modes(Problem p, int64_t batch, hipStream_t s, int am, bool b_kcontig) {
   // The pipeline moves whole 16-byte chunks along K (k % 4 == 0; rows are
   // 16-byte aligned on every caller's path) at 32-bit byte offsets, and a
-  // conv's 32-wide K tile has to lie inside one filter tap.
+  // conv's 32-wide K tile has to lie inside one filter tap, with no padded
+  // channels (it would read them).
   constexpr int64_t kMaxBytes = int64_t{1} << 31;
   if (batch == 1 && b_kcontig && p.k % 4 == 0 && p.a_bytes > 0 && p.a_bytes < kMaxBytes && p.b_bytes > 0 &&
       p.b_bytes < kMaxBytes && !switches().disable_dma) {
-    const bool tap = am == kConv && p.c_pack % 32 == 0;
-    const int tile = am == kDenseK || tap ? ks_tile(p, batch, device_cus()) : 0;
+    const bool tap = am == kConv && p.c_pack % 32 == 0 && p.cc == p.c_pack;
+    const int tile = am == kDenseK || tap ? ks_tile(p, batch, device_cus(), 4) : 0;
     if (tile) return launch_ks_f32(p, s, tap ? kConvTap : kDenseK, tile);
     if (am == kDenseK) return launch_f32_dma<kDenseK>(p, s);
     if (tap) return launch_f32_dma<kConvTap>(p, s);

@@ -2252,6 +2252,13 @@ __global__ void __launch_bounds__(NW * 64) mfma_gemm_dma_kernel(Problem p) {
     constexpr int N_DSR = KS * (TM + TN) * (Mma::kStep == 8 ? 2 : 1);
     constexpr int PER = N_MFMA / N_DSR;
     vec av[2][KS][TM], bv[2][KS][TN];
+    // fp32: the odd K steps sum apart, so a long K rounds in two chains of
+    // half its length.
+    acc_t acc_odd[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) acc_odd[i][j] = acc_t{0, 0, 0, 0};
     auto read_frags = [&](auto set_c, int stage) {
       constexpr int SET = decltype(set_c)::value;
       const uint8_t* As = smem + stage * STAGE;
@@ -2296,7 +2303,10 @@ __global__ void __launch_bounds__(NW * 64) mfma_gemm_dma_kernel(Problem p) {
       // between every PER MFMAs of tile kt.
       read_frags(std::integral_constant<int, SET ^ 1>{}, static_cast<int>((kt + 1) % S));
 #pragma unroll
-      for (int q = 0; q < KS; ++q) mma_step<Mma, TM, TN>(acc, av[SET][q], bv[SET][q]);
+      for (int q = 0; q < KS; ++q) {
+        if constexpr (std::is_same<Mma, MmaF32>::value) mma_step<Mma, TM, TN>(q ? acc_odd : acc, av[SET][q], bv[SET][q]);
+        else mma_step<Mma, TM, TN>(acc, av[SET][q], bv[SET][q]);
+      }
 #pragma unroll
       for (int g = 0; g < N_DSR; ++g) {
         __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);    // one LDS read
@@ -2308,6 +2318,12 @@ __global__ void __launch_bounds__(NW * 64) mfma_gemm_dma_kernel(Problem p) {
     for (int64_t kt = 0; kt < ktiles; kt += 2) {
       body(std::integral_constant<int, 0>{}, kt);
       if (kt + 1 < ktiles) body(std::integral_constant<int, 1>{}, kt + 1);
+    }
+    if constexpr (std::is_same<Mma, MmaF32>::value) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[i][j] += acc_odd[i][j];
     }
   } else {
 #pragma unroll
@@ -2555,19 +2571,22 @@ inline int device_cus() {
 
 // Whether the small-output kernel takes this GEMM or tap-uniform conv, and on
 // which tile (gemm_ks.h; 0 = no, 1 = 16 x 32, 2 = 32 x 32): outputs of at
-// most one 16 x 32 tile, or two 32 x 32 tiles, per CU.  Measured on 256 CUs
-// against the best shared-tile kernel (fp16, us): 333 x 512 x 2048 (M x N x
-// K) 5.8 against 12.2, 200 x 2304 x 768 (504 tiles of 32 x 32) 5.9 against
-// 7.4, 1000 x 512 x 2048 (512 tiles) 9.5 against 12.7; past the line 333 x
-// 2048 x 512 (704 tiles) 7.7 against 6.3.  16 x 32 over 32 x 32 where both
-// fit: 200 x 512 x 2048 5.1 against 5.8, in fp32 (MFMA-bound: twice the CUs)
-// 9.1 against 13.6.  Row-major outputs without the row_max side output only.
-inline int ks_tile(const Problem& p, int64_t batch, int cus) {
+// most one 16 x 32 tile, or two 32 x 32 tiles, per CU -- four where K is at
+// least 6 KB per row, which the shared tiles walk at 0.5 us per 128 bytes.
+// Measured on 256 CUs against the best shared-tile kernel (M x N x K, us):
+// 333 x 512 x 2048 5.5 / 12.2, 200 x 2304 x 768 (504 tiles of 32 x 32) 5.4 /
+// 7.4, 1000 x 512 x 2048 (512) 9.0 / 12.7; past the line 333 x 2048 x 512
+// (704) 7.7 / 6.3 and 2048 x 512 x 2048 (1024) 15.9 / 12.5, but 1000 x 768 x
+// 3072 (768) 17.2 / 26.3.  16 x 32 over 32 x 32 where both fit: 200 x 512 x
+// 2048 4.7 / 5.3, in fp32 (MFMA-bound: twice the CUs) 8.7 / 13.2.  Row-major
+// outputs without the row_max side output only.
+inline int ks_tile(const Problem& p, int64_t batch, int cus, int elem_bytes) {
   if (batch != 1 || p.out_nchw || p.epi.row_max != nullptr || switches().disable_dma || p.a_bytes <= 0 ||
       p.b_bytes <= 0 || p.a_bytes >= (int64_t{1} << 31) || p.b_bytes >= (int64_t{1} << 31))
     return 0;
   if (ceil_div(p.m, 16) * ceil_div(p.n, 32) <= cus) return 1;
-  return ceil_div(p.m, 32) * ceil_div(p.n, 32) <= 2 * cus ? 2 : 0;
+  const int64_t tiles32 = ceil_div(p.m, 32) * ceil_div(p.n, 32);
+  return tiles32 <= 2 * cus || (tiles32 <= 4 * cus && p.k * elem_bytes >= 6144) ? 2 : 0;
 }
 int launch_ks_16(Problem p, hipStream_t s, int in_dtype, int am, int tile);          // gemm_ks_16.hip
 int launch_ks_i8(Problem p, hipStream_t s, int mode, int out_dtype, int tile);       // gemm_ks_8.hip
@@ -2704,7 +2723,7 @@ int launch_h(Problem p, int64_t batch, hipStream_t s, int in_dtype) {
       const int cus = device_cus();
       // (Convs of at most 64 outputs keep the K-ordered kernel: the 64-channel
       // band kernel is bit-identical to it at every size.)
-      const int ks = AM == kConvTap && p.n <= 64 ? 0 : ks_tile(p, batch, cus);
+      const int ks = AM == kConvTap && p.n <= 64 ? 0 : ks_tile(p, batch, cus, 2);
       if (ks) return launch_ks_16(p, s, in_dtype, AM, ks);
       if (const int tile = mid_tile(p, batch, cus, AM, 2)) return launch_mid_16(p, s, in_dtype, AM, tile);
     }
@@ -2725,7 +2744,7 @@ int launch_h_any(Problem p, int64_t batch, hipStream_t s, int in_dtype) {
 template <typename TO>
 int launch_fp8(Problem p, hipStream_t s) {
   const int cus = device_cus();
-  if (const int tile = ks_tile(p, 1, cus)) return launch_ks_f8(p, s, p.out_dtype, tile);
+  if (const int tile = ks_tile(p, 1, cus, 1)) return launch_ks_f8(p, s, p.out_dtype, tile);
   if (const int tile = mid_tile(p, 1, cus, kDenseK, 1)) return launch_mid_f8(p, s, p.out_dtype, tile);
   dim3 grid;
   if (dma_eligible(p, 1, kDenseK) && big_tile_wins(p, device_cus(), sizeof(TO), false)) {

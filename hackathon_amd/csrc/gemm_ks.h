@@ -180,6 +180,35 @@ __global__ void __launch_bounds__(KW * 64) gemm_ks_kernel(Problem p) {
     if (AM == kConvTap) advance(KW * BK);
   };
 
+  // This thread's four output columns (at most one such piece per thread).
+  // For the common epilogue its operands -- residual, bias, E4M3 scales -- are
+  // loaded here, ahead of the operands, so that no memory round trip is left
+  // after the main loop.
+  constexpr int NC = BN / 4;
+  static_assert(BM * NC <= KW * 64, "one piece per thread");
+  const int o_row = tid / NC, o_col = tid % NC * 4;
+  const int64_t om = m0 + o_row, on = n0 + o_col;
+  const bool o_live = tid < BM * NC && om < p.m && on < p.n;
+  TO* out = static_cast<TO*>(p.out);
+  const TO* resp = static_cast<const TO*>(p.epi.residual);
+  constexpr uintptr_t kA = 4 * sizeof(TO) - 1;
+  const bool vec_ok = p.ldo % 4 == 0 && (reinterpret_cast<uintptr_t>(out) & kA) == 0 &&
+                      (reinterpret_cast<uintptr_t>(resp) & kA) == 0;
+  const bool wide = vec_ok && on + 4 <= p.n;
+  const bool simple = !Mma::kInt && wide && epilogue_is_simple(kernel_arg<Problem>(), vec_ok, true);
+  float res[4] = {0.f, 0.f, 0.f, 0.f}, row_scale = 1.0f;
+  float4 bias4 = make_float4(0.f, 0.f, 0.f, 0.f), col_scale = make_float4(1.f, 1.f, 1.f, 1.f);
+  if constexpr (!Mma::kInt) {
+    if (o_live && simple) {
+      if (resp) Elem<TO>::load4(resp + om * p.ldo + on, res);
+      if (p.epi.bias_mode == 2) bias4 = *reinterpret_cast<const float4*>(static_cast<const float*>(p.epi.bias) + on);
+      if constexpr (Mma::kScaled) {
+        row_scale = p.a_rows[om];
+        col_scale = *reinterpret_cast<const float4*>(p.b_scale + on);
+      }
+    }
+  }
+
   acc_t acc[TM][TN];
 #pragma unroll
   for (int i = 0; i < TM; ++i)
@@ -227,33 +256,40 @@ __global__ void __launch_bounds__(KW * 64) gemm_ks_kernel(Problem p) {
       *reinterpret_cast<float4*>(part + (16 * i + l16) * SS + 16 * j + 4 * lg) =
           __builtin_bit_cast(float4, acc[i][j]);  // C^T accumulators: row l16, columns 4 lg + r
   __syncthreads();
-  TO* out = static_cast<TO*>(p.out);
-  const TO* resp = static_cast<const TO*>(p.epi.residual);
-  constexpr uintptr_t kA = 4 * sizeof(TO) - 1;
-  const bool vec_ok = p.ldo % 4 == 0 && (reinterpret_cast<uintptr_t>(out) & kA) == 0 &&
-                      (reinterpret_cast<uintptr_t>(resp) & kA) == 0;
-  const QuantDiv qd(Mma::kInt ? p.q_scale : 1.0f);
-  constexpr int NC = BN / 4;
-#pragma unroll 1
-  for (int c = tid; c < BM * NC; c += KW * 64) {
-    const int row = c / NC, col = c % NC * 4;
-    const float* src = stage + row * SS + col;
-    float4 v = *reinterpret_cast<const float4*>(src);
+  if (!o_live) return;
+  const float* src = stage + o_row * SS + o_col;
+  float4 v = *reinterpret_cast<const float4*>(src);
 #pragma unroll
-    for (int w = 1; w < KW; ++w) {
-      const float4 u = *reinterpret_cast<const float4*>(src + w * BM * SS);
-      if constexpr (Mma::kInt) {
-        v = float4{__int_as_float(__float_as_int(v.x) + __float_as_int(u.x)),
-                   __int_as_float(__float_as_int(v.y) + __float_as_int(u.y)),
-                   __int_as_float(__float_as_int(v.z) + __float_as_int(u.z)),
-                   __int_as_float(__float_as_int(v.w) + __float_as_int(u.w))};
-      } else {
-        v = float4{v.x + u.x, v.y + u.y, v.z + u.z, v.w + u.w};
-      }
+  for (int w = 1; w < KW; ++w) {
+    const float4 u = *reinterpret_cast<const float4*>(src + w * BM * SS);
+    if constexpr (Mma::kInt) {
+      v = float4{__int_as_float(__float_as_int(v.x) + __float_as_int(u.x)),
+                 __int_as_float(__float_as_int(v.y) + __float_as_int(u.y)),
+                 __int_as_float(__float_as_int(v.z) + __float_as_int(u.z)),
+                 __int_as_float(__float_as_int(v.w) + __float_as_int(u.w))};
+    } else {
+      v = float4{v.x + u.x, v.y + u.y, v.z + u.z, v.w + u.w};
     }
-    const int64_t m = m0 + row, n = n0 + col;
-    if (m < p.m && n < p.n) ks_finish4<Mma, TO>(v, m, n, vec_ok && n + 4 <= p.n, out, resp, qd);
   }
+  if constexpr (!Mma::kInt) {
+    if (simple) {  // ((acc + bias) + residual), then the activation: apply_epilogue's arithmetic
+      const float acc4[4] = {v.x, v.y, v.z, v.w}, b4[4] = {bias4.x, bias4.y, bias4.z, bias4.w};
+      const float s4[4] = {col_scale.x, col_scale.y, col_scale.z, col_scale.w};
+      const int act = p.epi.act;
+      const float c0 = p.epi.imm[0], c1 = p.epi.imm[1], c2 = p.epi.imm[2];
+      const bool gstd = gelu_std_ok(c0, c1, c2);
+      float y[4];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const float t = ((Mma::kScaled ? (acc4[c] * row_scale) * s4[c] : acc4[c]) + b4[c]) + res[c];
+        y[c] = act == 1 ? fmaxf(t, 0.0f) : act == 2 ? gelu_act(t, c0, c1, c2, gstd) : t;
+      }
+      Elem<TO>::store4(out + om * p.ldo + on, y);
+      return;
+    }
+  }
+  const QuantDiv qd(Mma::kInt ? p.q_scale : 1.0f);
+  ks_finish4<Mma, TO>(v, om, on, wide, out, resp, qd);
 }
 
 // Tiles of launch_ks_*: 1 = 16 x 32 with eight waves, 2 = 32 x 32 with four.
