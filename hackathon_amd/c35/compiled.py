@@ -1111,9 +1111,11 @@ class CompiledPlan:
         self._finish_residual(st, out)
         mm = code
         # GEMMs with few output tiles run on small tiles that split K inside
-        # one launch (c3h_gemm).  Only a 16-bit output of a single 128 x 128
-        # tile is still split over two launches.
-        splits = self._splitk(m, n, k) if code != _lib.F32 and m <= 128 and n <= 128 else 1
+        # one launch (c3h_gemm).  Still split over two launches: an fp16 output
+        # of a single 128 x 128 tile, and bf16, where another order of the sums
+        # moves the argmax of nearly tied logits on about 1 % of positions.
+        split = code == _lib.BF16 or (code == _lib.F16 and m <= 128 and n <= 128)
+        splits = self._splitk(m, n, k) if split else 1
         if splits > 1:
             self._gemm_splitk(node, a2, w, out, st, m, n, k, splits, alpha, beta, bmode, in_code=code)
             return
