@@ -6,8 +6,8 @@
 // in parallel, and gemm.hip holds the C entry points.
 //
 //   fp32  : v_mfma_f32_16x16x4_f32   (the reference's fp32 policy)
-//   bf16  : v_mfma_f32_16x16x32_bf16 (config 3)
-//   f16   : v_mfma_f32_16x16x32_f16  (config 4)
+//   bf16  : v_mfma_f32_16x16x32_bf16
+//   f16   : v_mfma_f32_16x16x32_f16
 //
 // A 256-thread workgroup (4 wave64s) computes a BM x BN macro tile; each wave
 // owns a (BM/WM) x (BN/WN) sub-tile of 16x16 MFMA tiles.  A and B tiles are
