@@ -2569,20 +2569,21 @@ inline int device_cus() {
   return cus;
 }
 
-// Whether the small-output kernel takes this GEMM or tap-uniform conv, and on
+// Whether a small-output kernel takes this GEMM or tap-uniform conv, and on
 // which tile (gemm_ks.h; 0 = no, 1 = 16 x 32, 2 = 32 x 32): outputs of at
 // most one 16 x 32 tile, or two 32 x 32 tiles, per CU -- four where K is at
 // least 6 KB per row, which the shared tiles walk at 0.5 us per 128 bytes.
 // Measured on 256 CUs against the best shared-tile kernel (M x N x K, us):
-// 333 x 512 x 2048 5.5 / 12.2, 200 x 2304 x 768 (504 tiles of 32 x 32) 5.4 /
-// 7.4, 1000 x 512 x 2048 (512) 9.0 / 12.7; past the line 333 x 2048 x 512
+// 333 x 512 x 2048 5.5 / 12.2, 200 x 2304 x 768 (504 tiles of 32 x 32) 5.2 /
+// 7.4, 1000 x 512 x 2048 (512) 8.8 / 12.7; past the line 333 x 2048 x 512
 // (704) 7.7 / 6.3 and 2048 x 512 x 2048 (1024) 15.9 / 12.5, but 1000 x 768 x
-// 3072 (768) 17.2 / 26.3.  16 x 32 over 32 x 32 where both fit: 200 x 512 x
-// 2048 4.7 / 5.3, in fp32 (MFMA-bound: twice the CUs) 8.7 / 13.2.  Row-major
+// 3072 (768) 15.9 / 26.3.  16 x 32 over 32 x 32 where both fit: 200 x 512 x
+// 2048 4.5 / 5.3, in fp32 (MFMA-bound: twice the CUs) 8.7 / 13.2.  Row-major
 // outputs without the row_max side output only.
 inline int ks_tile(const Problem& p, int64_t batch, int cus, int elem_bytes) {
-  if (batch != 1 || p.out_nchw || p.epi.row_max != nullptr || switches().disable_dma || p.a_bytes <= 0 ||
-      p.b_bytes <= 0 || p.a_bytes >= (int64_t{1} << 31) || p.b_bytes >= (int64_t{1} << 31))
+  if (batch != 1 || p.out_nchw || p.epi.row_max != nullptr || switches().disable_dma ||
+      switches().disable_smalltile || p.a_bytes <= 0 || p.b_bytes <= 0 || p.a_bytes >= (int64_t{1} << 31) ||
+      p.b_bytes >= (int64_t{1} << 31))
     return 0;
   if (ceil_div(p.m, 16) * ceil_div(p.n, 32) <= cus) return 1;
   const int64_t tiles32 = ceil_div(p.m, 32) * ceil_div(p.n, 32);
@@ -2607,7 +2608,7 @@ int launch_ks_f32(Problem p, hipStream_t s, int am, int tile);                  
 // 12.3, 37 (227 tiles) 16.9 / 16.5 / 14.5, 64 (392) 20.8 / 26.1 / 29.4.  The
 // K order is that of the other tiles: bit-identical results.
 inline int mid_tile(const Problem& p, int64_t batch, int cus, int am, int elem_bytes) {
-  if (!dma_eligible(p, batch, am)) return 0;
+  if (switches().disable_smalltile || !dma_eligible(p, batch, am)) return 0;
   if (ceil_div(p.m, 64) * ceil_div(p.n, 64) <= 2 * cus) return 1;
   const int64_t tiles128 = ceil_div(p.m, 128) * ceil_div(p.n, 128);
   return tiles128 <= cus || (am == kDenseK && p.k * elem_bytes <= 1024 && 2 * tiles128 <= 3 * cus) ? 2 : 0;

@@ -9,10 +9,10 @@ template <typename Mma, typename T>
 int launch_ks_type(Problem p, hipStream_t s, int am, int tile) {
   const bool f32 = p.out_dtype == C3H_F32;
   if (am == kConvTap)
-    return f32 ? launch_ks_tile<Mma, float, kConvTap>(p, s, tile, "conv_ks")
-               : launch_ks_tile<Mma, T, kConvTap>(p, s, tile, "conv_ks");
-  return f32 ? launch_ks_tile<Mma, float, kDenseK>(p, s, tile, "gemm_ks")
-             : launch_ks_tile<Mma, T, kDenseK>(p, s, tile, "gemm_ks");
+    return f32 ? launch_ordered_tile<Mma, float, kConvTap>(p, s, tile, "conv_small")
+               : launch_ordered_tile<Mma, T, kConvTap>(p, s, tile, "conv_small");
+  return f32 ? launch_ordered_tile<Mma, float, kDenseK>(p, s, tile, "gemm_small")
+             : launch_ordered_tile<Mma, T, kDenseK>(p, s, tile, "gemm_small");
 }
 }  // namespace
 

@@ -13,9 +13,9 @@ int launch_ks_i8(Problem p, hipStream_t s, int mode, int out_dtype, int tile) {
 }
 
 int launch_ks_f8(Problem p, hipStream_t s, int out_dtype, int tile) {
-  if (out_dtype == C3H_F32) return launch_ks_tile<MmaF8, float, kDenseK>(p, s, tile, "gemm_fp8_ks");
-  if (out_dtype == C3H_BF16) return launch_ks_tile<MmaF8, bf16_t, kDenseK>(p, s, tile, "gemm_fp8_ks");
-  return launch_ks_tile<MmaF8, f16_t, kDenseK>(p, s, tile, "gemm_fp8_ks");
+  if (out_dtype == C3H_F32) return launch_ordered_tile<MmaF8, float, kDenseK>(p, s, tile, "gemm_fp8_small");
+  if (out_dtype == C3H_BF16) return launch_ordered_tile<MmaF8, bf16_t, kDenseK>(p, s, tile, "gemm_fp8_small");
+  return launch_ordered_tile<MmaF8, f16_t, kDenseK>(p, s, tile, "gemm_fp8_small");
 }
 
 int launch_ks_f32(Problem p, hipStream_t s, int am, int tile) {

@@ -495,7 +495,13 @@ typedef struct {
  * (broadcast).  Replaces kernel_matmul (kernel_registry.py:318-358) and the
  * gemm epilogue kernel (c35/engine.py:722-844).  in_dtype applies to A and B
  * (F32 -> fp32 MFMA 16x16x4; F16/BF16 -> MFMA 16x16x32 with fp32
- * accumulation); out_dtype F32/F16/BF16. */
+ * accumulation); out_dtype F32/F16/BF16.
+ * Order of the sums, here and in c3h_conv2d, c3h_gemm_fp8 and
+ * c3h_gemm_w4a16: 16-bit and E4M3 operands sum K in order whatever the
+ * shape, so an output's bits do not depend on how many rows or columns the
+ * call has.  fp32 operands sum in an order fixed for a shape, but outputs of
+ * few tiles split K over the waves of a workgroup: there the last bits of a
+ * row can depend on m and n. */
 typedef struct {
   const void* a;
   const void* b;
@@ -802,9 +808,7 @@ int c3h_quantize_mxfp4(const c3h_mxfp4_quant_args* a, void* stream);
  * W[n,k] = E2M1(codes) * 2^(scales[n][k/32] - 127) widened to fp16 in
  * registers (exact under c3h_quantize_mxfp4's exponent range), fp16 MFMA
  * with fp32 accumulation, and the common epilogue into fp32 or fp16.
- * Equals, bit for bit, the fp16 GEMM of the dequantized weights that sums K
- * in order (c3h_gemm's result, except where it splits the K of an output of
- * few tiles over the waves of a workgroup).  k % 32 == 0,
+ * Equals c3h_gemm on the dequantized fp16 weights bit for bit.  k % 32 == 0,
  * lda % 8 == 0, ldb (bytes) % 4 == 0 and >= k/2, ldbs >= k/32; A 16-byte
  * aligned; A, codes and scales each below 2^31 bytes. */
 typedef struct {

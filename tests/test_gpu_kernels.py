@@ -1682,12 +1682,14 @@ def test_conv_fp32_pipeline_edges(gpu, n, h, w, c, o, ks, stride, nchw):
 @pytest.mark.parametrize("kind", ["fp32", "fp16", "bf16", "fp8", "int8"])
 @pytest.mark.parametrize("m,n,k,ldo,form", [
     (1, 10, 64, 10, "relu"), (17, 33, 144, 40, "program"), (16, 32, 2048, 32, "gelu"),   # 16 x 32 tiles
+    (130, 40, 16, 40, "scaled"), (40, 300, 784, 300, "scaled"),
     (515, 289, 272, 292, "relu"), (1000, 512, 1040, 512, "gelu"), (700, 770, 6144, 772, "program")])  # 32 x 32
 def test_small_output_gemm_matches_the_general_kernel(gpu, kind, m, n, k, ldo, form):
-    """GEMMs of few output tiles split K over the waves of a workgroup: one row, ragged edges, fewer K tiles
-    than waves, a partial last K tile and strided output rows, against the register-staged kernel
-    (C3H_DISABLE_DMA).  int8 codes are equal; a float dot product of K terms moves by at most K 2^-23 of
-    sum |a b| between two summation orders, plus the output type's rounding."""
+    """GEMMs of few output tiles on their small tiles: one row, ragged edges, fewer K tiles than waves, a partial
+    last K tile and strided output rows, against the 128 x 128 tiles (C3H_DISABLE_SMALLTILE) and the
+    register-staged kernel (C3H_DISABLE_DMA).  16-bit and E4M3 operands sum K in order on every tile: the same
+    bits.  int8 codes are equal.  fp32 splits K over the waves of a workgroup: a dot product of K terms moves by
+    at most K 2^-23 of sum |a b| between two summation orders, plus the output's rounding."""
     from hackathon_amd import _lib
     from hackathon_amd.c35 import engine as E
     from hackathon_amd.device import DeviceArray
@@ -1696,7 +1698,7 @@ def test_small_output_gemm_matches_the_general_kernel(gpu, kind, m, n, k, ldo, f
     if kind == "fp8":  # finite E4M3 codes of magnitudes up to 1.875
         a, b = (rng.integers(0, 0x40, s, dtype=np.uint8) | (rng.integers(0, 2, s, dtype=np.uint8) << 7) for s in
                 ((m, k), (n, k)))
-        size, out_np = 2.0 ** 2 * k * np.ones((m, n)), np.float16
+        out_np = np.float16
     elif kind == "int8":
         a, b = (rng.integers(-128, 128, s, dtype=np.int8) for s in ((m, k), (n, k)))
         out_np = np.int8
@@ -1707,6 +1709,7 @@ def test_small_output_gemm_matches_the_general_kernel(gpu, kind, m, n, k, ldo, f
     bias, scale = _dev(rng.standard_normal(n, dtype=np.float32)), _dev(rng.random(max(m, n), dtype=np.float32) + 0.5)
     prog = [(_lib.EW_MUL, 0, 2, 0.0), (_lib.EW_ADD, 1, 0, 0.0)]
     epi = E.epilogue(bias=bias, bias_mode=2, **{"relu": dict(act=1), "gelu": dict(act=2, imm=[math.sqrt(2.0), 1.0, 0.5]),
+                                                "scaled": dict(alpha=0.7, beta=0.3),
                                                 "program": dict(program=prog, imm=[0.25])}[form])
     ad, bd = _dev(a), _dev(b)
 
@@ -1725,24 +1728,65 @@ def test_small_output_gemm_matches_the_general_kernel(gpu, kind, m, n, k, ldo, f
         _lib.launch(g)
         return out.get()
 
-    got, want = run(), switches.with_switch("C3H_DISABLE_DMA", "1", run)
-    if kind == "int8":
-        np.testing.assert_array_equal(got, want)
-        return
-    got, want = (x if kind in ("fp32", "fp8") else _from16(x, kind) for x in (got, want))
-    got, want = got.astype(np.float64), want.astype(np.float64)
-    assert not got[:, n:].any()
-    # slopes of the epilogue forms are at most 1.25; row and column scales of fp8 at most 1.5 each
-    bound = 1.25 * (2.25 if kind == "fp8" else 1.0) * k * 2.0 ** -23 * size
-    ulp = {"fp32": 2.0 ** -22, "bf16": 2.0 ** -7}.get(kind, 2.0 ** -10)
-    assert np.all(np.abs(got - want)[:, :n] <= bound + ulp * np.abs(want[:, :n]) + 2.0 ** -24)
+    got = run()
+    assert got[:, :n].any() and not got[:, n:].any()
+    for switch in ("C3H_DISABLE_SMALLTILE", "C3H_DISABLE_DMA"):
+        want = switches.with_switch(switch, "1", run)
+        if kind == "fp32":  # slopes of the epilogue forms are at most 1.25
+            bound = 1.25 * k * 2.0 ** -23 * size + 2.0 ** -22 * np.abs(want[:, :n]) + 2.0 ** -24
+            assert np.all(np.abs(got.astype(np.float64) - want)[:, :n] <= bound)
+        else:
+            np.testing.assert_array_equal(got.view(np.uint8), want.view(np.uint8), err_msg=switch)
+
+
+@pytest.mark.parametrize("kind", ["fp16", "bf16", "fp8", "fp4"])
+@pytest.mark.parametrize("n,k", [(512, 2048), (1000, 512), (30, 96)])
+def test_gemm_rows_do_not_depend_on_the_row_count(gpu, kind, n, k):
+    """Calls of 1, 40, 333 and 3000 rows take different tiles; a row's bits are the same in all of them."""
+    from hackathon_amd import _lib
+    from hackathon_amd.c35 import engine as E
+    from hackathon_amd.device import DeviceArray
+
+    rng = np.random.default_rng(n + k)
+    kk = -(-k // 32) * 32
+    x = rng.standard_normal((3000, kk), dtype=np.float32)
+    if kind == "fp8":
+        ad, bd = (_dev(rng.integers(0, 0x60, s, dtype=np.uint8) | (rng.integers(0, 2, s, dtype=np.uint8) << 7)) for s in
+                  ((3000, kk), (n, kk)))
+        scale = _dev(rng.random(3000, dtype=np.float32) + 0.5)
+    else:
+        ad = _dev(_bits(x, "bf16" if kind == "bf16" else "fp16")[0])
+        bd = _dev(_bits(rng.standard_normal((n, kk), dtype=np.float32), "bf16" if kind == "bf16" else "fp16")[0])
+    codes, exps = _dev(rng.integers(0, 256, (n, kk // 2), dtype=np.uint8)), _dev(rng.integers(120, 130, (n, kk // 32), dtype=np.uint8))
+    bias = _dev(rng.standard_normal(n, dtype=np.float32))
+
+    def rows(m):
+        out = DeviceArray.from_host(np.zeros((m, n), np.float32))
+        g = {"fp8": _lib.Fp8GemmArgs, "fp4": _lib.W4A16GemmArgs}.get(kind, _lib.GemmArgs)()
+        g.a, g.out, g.m, g.n, g.k, g.lda, g.ldo, g.out_dtype = ad.ptr, out.ptr, m, n, kk, kk, n, _lib.F32
+        g.epi = E.epilogue(bias=bias, bias_mode=2, act=1)
+        if kind == "fp4":
+            g.b_codes, g.b_scales, g.ldb, g.ldbs = codes.ptr, exps.ptr, kk // 2, kk // 32
+        else:
+            g.b, g.ldb = bd.ptr, kk
+        if kind == "fp8":
+            g.a_scale, g.b_scale = scale.ptr, scale.ptr
+        elif kind != "fp4":
+            g.batch, g.trans_b, g.in_dtype = 1, 1, ad.code
+        _lib.launch(g)
+        return out.get()
+
+    want = rows(3000)
+    assert want.any()
+    for m in (1, 40, 333):
+        np.testing.assert_array_equal(rows(m), want[:m], err_msg=f"{m} rows")
 
 
 @pytest.mark.parametrize("kind,c", [("fp32", 32), ("bf16", 64), ("fp16", 192)])
 @pytest.mark.parametrize("n,hw,o,ks,stride", [(1, 7, 72, 3, 1), (2, 5, 512, 1, 2), (3, 14, 100, 3, 2)])
 def test_small_output_conv_matches_the_general_kernel(gpu, kind, c, n, hw, o, ks, stride):
-    """Tap-uniform convs of few output tiles (each wave of a workgroup walks every KW-th K tile, across filter
-    taps), with residual and ReLU, against the register-staged kernel (same bound as the GEMMs)."""
+    """Tap-uniform convs of few output tiles, their K tiles across filter taps, with residual and ReLU, against
+    the 128 x 128 tiles and the register-staged kernel: the same bits in 16 bits, the GEMMs' bound in fp32."""
     from hackathon_amd import _lib
     from hackathon_amd.c35 import engine as E
     from hackathon_amd.device import DeviceArray
@@ -1765,11 +1809,15 @@ def test_small_output_conv_matches_the_general_kernel(gpu, kind, c, n, hw, o, ks
         _lib.launch(a)
         return out.get()
 
-    got, want = run(), switches.with_switch("C3H_DISABLE_DMA", "1", run)
-    got, want = ((x if kind == "fp32" else _from16(x, kind)).astype(np.float64) for x in (got, want))
+    got = run()
     k = ks * ks * c  # |a b| sums to about 0.64 k on standard normals; 2 k bounds it
-    ulp = {"fp32": 2.0 ** -22, "bf16": 2.0 ** -7, "fp16": 2.0 ** -10}[kind]
-    assert np.all(np.abs(got - want) <= 2 * k * k * 2.0 ** -23 + ulp * np.abs(want)) and want.any()
+    for switch in ("C3H_DISABLE_SMALLTILE", "C3H_DISABLE_DMA"):
+        want = switches.with_switch(switch, "1", run)
+        assert want.any()
+        if kind == "fp32":
+            assert np.all(np.abs(got.astype(np.float64) - want) <= 2 * k * k * 2.0 ** -23 + 2.0 ** -22 * np.abs(want))
+        else:
+            np.testing.assert_array_equal(got.view(np.uint16), want.view(np.uint16), err_msg=switch)
 
 
 @pytest.mark.parametrize("mask_kind", [0, 1, 2])
