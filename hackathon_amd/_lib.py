@@ -34,7 +34,8 @@ OP_NOP, OP_EVENT_RECORD, OP_EVENT_WAIT, OP_COPY = 0, 1, 2, 3
 OP_FILL, OP_CAST, OP_EW, OP_STRIDED_COPY, OP_REDUCE, OP_SOFTMAX, OP_LAYERNORM, OP_BATCHNORM, \
     OP_GATHER, OP_ARGMAX, OP_IM2COL, OP_LAYOUT, OP_MAXPOOL, OP_GEMM, OP_CONV, OP_ATTN_SCORES, \
     OP_FLASH, OP_QUANTIZE, OP_QGEMM, OP_DEQUANTIZE, OP_BNFOLD, OP_PACK, OP_CONV_POOL, OP_QUANT_FP8, \
-    OP_GEMM_FP8, OP_SPLITK, OP_QUANT_MXFP4, OP_GEMM_W4A16, OP_ARGMAX_FINISH, OP_NONFINITE, OP_FLASH_F32 = range(10, 41)
+    OP_GEMM_FP8, OP_SPLITK, OP_QUANT_MXFP4, OP_GEMM_W4A16, OP_ARGMAX_FINISH, OP_NONFINITE, OP_FLASH_F32, \
+    OP_GEMM_SPLITK = range(10, 42)
 
 vp = C.c_void_p
 i32 = C.c_int32
@@ -228,6 +229,10 @@ class SplitKArgs(C.Structure):
                 ("out_dtype", i32), ("epi", Epilogue)]
 
 
+class GemmSplitKArgs(C.Structure):
+    _fields_ = [("gemm", GemmArgs), ("workspace", vp), ("workspace_bytes", i64), ("splits", i32), ("pad_", i32)]
+
+
 class ConvPoolArgs(C.Structure):
     _fields_ = [("x", vp), ("w", vp), ("bias", vp), ("out", vp)] + [(n, i32) for n in (
         "n", "c", "h", "w_", "o", "k_stride", "kh", "kw", "sh", "sw", "pad_top", "pad_left", "ho", "wo",
@@ -243,7 +248,8 @@ ABI_ORDER = [Props, FillArgs, CastArgs, EwArgs, CopyArgs, ReduceArgs, SoftmaxArg
              BatchNormArgs, BnFoldArgs, GatherArgs, ArgmaxArgs, Im2colArgs, LayoutArgs, PoolArgs,
              Epilogue, GemmArgs, ConvArgs, AttnScoresArgs, FlashArgs, QuantizeArgs, QGemmArgs,
              DequantizeArgs, Op, PackArgs, ConvPoolArgs, Fp8QuantArgs, Fp8GemmArgs,
-             SplitKArgs, Mxfp4QuantArgs, W4A16GemmArgs, ArgmaxFinishArgs, NonfiniteArgs]
+             SplitKArgs, Mxfp4QuantArgs, W4A16GemmArgs, ArgmaxFinishArgs, NonfiniteArgs,
+             GemmSplitKArgs]
 
 # Kernel entry points: name -> args struct (all take (const args*, void* stream)).
 KERNELS = {
@@ -258,6 +264,7 @@ KERNELS = {
     "c3h_quantize_fp8_rows": Fp8QuantArgs, "c3h_gemm_fp8": Fp8GemmArgs,
     "c3h_gemm_splitk_reduce": SplitKArgs, "c3h_quantize_mxfp4": Mxfp4QuantArgs,
     "c3h_gemm_w4a16": W4A16GemmArgs, "c3h_argmax_finish": ArgmaxFinishArgs, "c3h_nonfinite": NonfiniteArgs,
+    "c3h_gemm_splitk_launch": GemmSplitKArgs,
 }
 
 OP_KIND = {
@@ -270,7 +277,7 @@ OP_KIND = {
     BnFoldArgs: OP_BNFOLD, PackArgs: OP_PACK, ConvPoolArgs: OP_CONV_POOL,
     Fp8QuantArgs: OP_QUANT_FP8, Fp8GemmArgs: OP_GEMM_FP8, SplitKArgs: OP_SPLITK,
     Mxfp4QuantArgs: OP_QUANT_MXFP4, W4A16GemmArgs: OP_GEMM_W4A16, ArgmaxFinishArgs: OP_ARGMAX_FINISH,
-    NonfiniteArgs: OP_NONFINITE, FlashF32Args: OP_FLASH_F32,
+    NonfiniteArgs: OP_NONFINITE, FlashF32Args: OP_FLASH_F32, GemmSplitKArgs: OP_GEMM_SPLITK,
 }
 
 KERNEL_OF_ARGS = {v: k for k, v in KERNELS.items()}

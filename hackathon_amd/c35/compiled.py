@@ -1110,14 +1110,13 @@ class CompiledPlan:
         out = self._new(out_shape, self._out_dtype(st.final))
         self._finish_residual(st, out)
         mm = code
-        # GEMMs with few output tiles run on small tiles that split K inside
-        # one launch (c3h_gemm).  Still split over two launches: an fp16 output
-        # of a single 128 x 128 tile, and bf16, where another order of the sums
-        # moves the argmax of nearly tied logits on about 1 % of positions.
-        split = code == _lib.BF16 or (code == _lib.F16 and m <= 128 and n <= 128)
-        splits = self._splitk(m, n, k) if split else 1
+        # 16-bit GEMMs with few output tiles sum K in `splits` partials, added
+        # in order.  The partials are part of the result: another order moves
+        # the argmax of nearly tied logits on about 1 % of positions.  (fp32
+        # GEMMs of few tiles split K inside c3h_gemm.)
+        splits = self._splitk(m, n, k) if code != _lib.F32 else 1
         if splits > 1:
-            self._gemm_splitk(node, a2, w, out, st, m, n, k, splits, alpha, beta, bmode, in_code=code)
+            self._gemm_splitk(a2, w, out, st, m, n, k, splits, alpha, beta, bmode, code)
             return
 
         def build(r, a2=a2, w=w, out=out, st=st, m=m, n=n, k=k):
@@ -1150,32 +1149,25 @@ class CompiledPlan:
                 best = s
         return best
 
-    def _gemm_splitk(self, node, a2: Val, w: Val, out: Val, st: "_Epi", m: int, n: int, k: int, splits: int,
-                     alpha: float, beta: float, bmode, in_code: int = _lib.F32) -> None:
-        """Split-K: `splits` batched partial GEMMs over K/splits each into an fp32
-        workspace (fp32 accumulation for 16-bit operands too), then
-        c3h_gemm_splitk_reduce (fixed summation order + epilogue)."""
-        ks = k // splits
+    def _gemm_splitk(self, a2: Val, w: Val, out: Val, st: "_Epi", m: int, n: int, k: int, splits: int, alpha: float,
+                     beta: float, bmode, in_code: int) -> None:
+        """A GEMM whose K is summed as `splits` fp32 partials, added in order
+        before the epilogue (c3h_gemm_splitk: one launch that keeps them in
+        registers where its tiles take the shape, else batched partial GEMMs
+        into the workspace and a reduce; the same bits)."""
         part = self._new((splits, m, n), np.float32)
 
-        def gbuild(r, a2=a2, w=w, part=part):
-            g = _lib.GemmArgs()
-            g.a, g.b, g.out = self._ptr(a2, r), self._ptr(w, r), self._ptr(part, r)
-            g.m, g.n, g.k, g.lda, g.ldb, g.ldo, g.batch = m, n, ks, k, k, n, splits
-            g.stride_a, g.stride_b, g.stride_out = ks, ks, m * n
-            g.trans_a, g.trans_b, g.in_dtype, g.out_dtype = 0, 1, in_code, _lib.F32
-            g.epi.alpha, g.epi.beta = 1.0, 1.0
-            return g
-        self._emit(f"gemm:{node.op_type}", gbuild, [a2, w], [part], flops=2.0 * m * n * k,
-                   info=f"M={m} N={n} K={k} in {splits} K splits")
-
-        def rbuild(r, part=part, out=out, st=st):
-            g = _lib.SplitKArgs()
-            g.partial, g.out = self._ptr(part, r), self._ptr(out, r)
-            g.m, g.n, g.ldo, g.splits, g.out_dtype = m, n, n, splits, dtype_code(out.dtype)
+        def build(r, a2=a2, w=w, part=part, out=out, st=st):
+            s = _lib.GemmSplitKArgs()
+            g = s.gemm
+            g.a, g.b, g.out = self._ptr(a2, r), self._ptr(w, r), self._ptr(out, r)
+            g.m, g.n, g.k, g.lda, g.ldb, g.ldo, g.batch = m, n, k, k, k, n, 1
+            g.trans_a, g.trans_b, g.in_dtype, g.out_dtype = 0, 1, in_code, dtype_code(out.dtype)
             self._fill_epi(g.epi, st, r, alpha, beta, bmode)
-            return g
-        self._emit("splitk_reduce", rbuild, [part] + self._epi_reads(st), [out])
+            s.workspace, s.workspace_bytes, s.splits = self._ptr(part, r), splits * m * n * 4, splits
+            return s
+        self._emit("splitk_reduce", build, [a2, w] + self._epi_reads(st), [part, out], flops=2.0 * m * n * k,
+                   skip_bytes=[part], info=f"M={m} N={n} K={k} in {splits} K splits")
         self.vals[st.final] = out
 
     def _op_FusedGemmEpilogue(self, node):

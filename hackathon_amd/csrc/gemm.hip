@@ -36,6 +36,22 @@ __global__ void __launch_bounds__(256) gemm_simple_kernel(Problem p) {
   outp[o] = apply_epilogue(kernel_arg<Problem>().epi, acc, m, n, p.n, res, bz * p.stride_bias);
 }
 
+void fill_dense(Problem& p, const c3h_gemm_args* a) {
+  memset(&p, 0, sizeof(p));
+  p.a = a->a; p.b = a->b; p.out = a->out;
+  p.m = a->m; p.n = a->n; p.k = a->k;
+  p.lda = a->lda; p.ldb = a->ldb; p.ldo = a->ldo;
+  p.stride_a = a->stride_a; p.stride_b = a->stride_b; p.stride_out = a->stride_out;
+  p.stride_bias = a->stride_bias; p.stride_res = a->stride_res;
+  p.trans_a = a->trans_a; p.trans_b = a->trans_b;
+  p.out_dtype = a->out_dtype;
+  p.epi = a->epi;
+  p.ho = 1; p.wo = 1;
+  const int es = dtype_size(a->in_dtype);
+  p.a_bytes = ((a->m - 1) * a->lda + a->k) * es;
+  p.b_bytes = ((a->n - 1) * a->ldb + a->k) * es;
+}
+
 }  // namespace
 
 extern "C" {
@@ -52,21 +68,7 @@ int c3h_gemm(const c3h_gemm_args* a, void* stream) {
   C3H_REQUIRE(a->k >= 1, "gemm: k must be >= 1 for a non-empty output");
   C3H_REQUIRE(a->ldo >= a->n, "gemm: ldo < n");
   Problem p;
-  memset(&p, 0, sizeof(p));
-  p.a = a->a; p.b = a->b; p.out = a->out;
-  p.m = a->m; p.n = a->n; p.k = a->k;
-  p.lda = a->lda; p.ldb = a->ldb; p.ldo = a->ldo;
-  p.stride_a = a->stride_a; p.stride_b = a->stride_b; p.stride_out = a->stride_out;
-  p.stride_bias = a->stride_bias; p.stride_res = a->stride_res;
-  p.trans_a = a->trans_a; p.trans_b = a->trans_b;
-  p.out_dtype = a->out_dtype;
-  p.epi = a->epi;
-  p.ho = 1; p.wo = 1;
-  {
-    const int es = dtype_size(a->in_dtype);
-    p.a_bytes = ((a->m - 1) * a->lda + a->k) * es;
-    p.b_bytes = ((a->n - 1) * a->ldb + a->k) * es;
-  }
+  fill_dense(p, a);
   int64_t tiles = ceil_div(a->m, 64) * ceil_div(a->n, 64);
   C3H_REQUIRE(tiles < (1LL << 31), "gemm: too many tiles");
   hipStream_t s = as_stream(stream);
@@ -203,9 +205,39 @@ int64_t splitk_partial_bytes(const c3h_gemm_args* a, int32_t splits) {
   return mn * splits * 4;
 }
 
+// Whether a split-K GEMM can keep its partial sums in registers: 16-bit
+// operands whose K/splits is whole 64-wide K tiles, on an output that a
+// small-output or 64-column tile takes (every output the compiled engine
+// splits).  Fills p and the tile: 1 / 2 of ks_tile, 3 / 4 for 1 / 2 of mid_tile.
+int splitk_in_registers(const c3h_gemm_args* a, int32_t splits, Problem& p) {
+  if ((a->in_dtype != C3H_BF16 && a->in_dtype != C3H_F16) || a->trans_a || !a->trans_b || splits < 2 ||
+      a->k / splits % 64 != 0 || a->lda % 8 != 0 || a->ldb % 8 != 0 || !aligned(a->a, 16) || !aligned(a->b, 16) ||
+      a->ldo < a->n || (a->out_dtype != C3H_F32 && a->out_dtype != a->in_dtype) || a->k >= (int64_t{1} << 31))
+    return 0;
+  fill_dense(p, a);
+  // An output over an operand needs the two launches: the partial GEMMs have
+  // read all of A and B before the reduce writes.
+  const uintptr_t out = reinterpret_cast<uintptr_t>(a->out);
+  const uintptr_t end = out + static_cast<uintptr_t>(((a->m - 1) * a->ldo + a->n) * dtype_size(a->out_dtype));
+  auto over = [&](const void* ptr, int64_t bytes) {
+    const uintptr_t at = reinterpret_cast<uintptr_t>(ptr);
+    return out < at + static_cast<uintptr_t>(bytes) && at < end;
+  };
+  if (over(a->a, p.a_bytes) || over(a->b, p.b_bytes)) return 0;
+  p.k_part = static_cast<int>(a->k / splits);
+  const int cus = device_cus();
+  if (const int tile = ks_tile(p, 1, cus, 2)) return tile;
+  const int mid = mid_tile(p, 1, cus, kDenseK, 2);
+  return mid ? 2 + mid : 0;
+}
+
 // The split-K GEMM over a given fp32 partial buffer (the caller has checked
 // its size): `splits` batched partial GEMMs over K/splits each, plain
-// epilogue, then the ordered reduce with a's epilogue.
+// epilogue, then the ordered reduce with a's epilogue -- or one launch that
+// forms the same partials and the same ordered sum in registers, where it can
+// (two launches / one, fp16, M x N x K in splits, us: 1 x 512 x 512 in 8 7.9 /
+// 3.3, 200 x 512 x 2048 in 32 20.0 / 5.3, 200 x 8192 x 512 in 4 27.3 / 7.8,
+// 1000 x 512 x 2048 in 16 24.0 / 9.4, 3000 x 768 x 768 in 3 26.0 / 13.3).
 int gemm_splitk_into(const c3h_gemm_args* a, int32_t splits, float* partial, hipStream_t s) {
   C3H_REQUIRE(a->batch == 1, "gemm_splitk: batch must be 1 (one GEMM split along K)");
   C3H_REQUIRE(splits >= 1 && splits <= 64, "gemm_splitk: splits %d outside [1, 64]", splits);
@@ -216,6 +248,9 @@ int gemm_splitk_into(const c3h_gemm_args* a, int32_t splits, float* partial, hip
   int rc = check_epilogue(a->epi);
   if (rc) return rc;
   if (a->m == 0 || a->n == 0) return C3H_OK;
+  Problem p;
+  if (const int tile = splitk_in_registers(a, splits, p))
+    return tile <= 2 ? launch_ks_16_part(p, s, a->in_dtype, tile) : launch_mid_16_part(p, s, a->in_dtype, tile - 2);
   const int64_t ks = a->k / splits;
   c3h_gemm_args g = *a;
   g.out = partial;
@@ -316,6 +351,11 @@ int c3h_gemm_splitk(const c3h_gemm_args* a, int32_t splits, void* workspace, siz
               workspace_bytes, static_cast<long long>(need));
   C3H_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 15) == 0, "gemm_splitk: workspace must be 16-byte aligned");
   return gemm_splitk_into(a, splits, static_cast<float*>(workspace), as_stream(stream));
+}
+
+int c3h_gemm_splitk_launch(const c3h_gemm_splitk_args* a, void* stream) {
+  C3H_REQUIRE(a != nullptr && a->workspace_bytes >= 0, "gemm_splitk: null args or bad workspace size");
+  return c3h_gemm_splitk(&a->gemm, a->splits, a->workspace, static_cast<size_t>(a->workspace_bytes), stream);
 }
 
 int c3h_gemm_fp8(const c3h_fp8_gemm_args* a, void* stream) {

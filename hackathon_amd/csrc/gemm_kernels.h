@@ -275,6 +275,7 @@ struct Problem {
   // E8M0 exponents [n][ldbs] of its 32-element blocks (bs_bytes in all)
   const uint8_t* b_blk;
   int64_t ldbs, bs_bytes;
+  int k_part;  // K of each partial sum of a split-K GEMM run in one launch
   c3h_epilogue epi;
 };
 
@@ -2064,8 +2065,12 @@ __device__ __forceinline__ void wait_vmcnt_groups(int64_t n) {
 // current one) and an MFMA phase, offset by one workgroup barrier, so on
 // every SIMD one wave multiplies while the other loads.  Same K order and
 // accumulation as the other forms: bit-identical results.
+//
+// PART (plain form): the accumulators are added to a total and restarted after
+// every p.k_part of K -- the fp32 partials and the ordered sum of a split-K
+// GEMM (splitk_reduce_kernel), with neither in memory.
 template <typename Mma, typename TO, int BM, int BN, int WM, int WN, int AM, int S, int NW = 4, bool RP = false,
-          bool PP = false>
+          bool PP = false, bool PART = false>
 __global__ void __launch_bounds__(NW * 64) mfma_gemm_dma_kernel(Problem p) {
   constexpr bool DIRECT = NW > 4;
   // The 160-row tile has no staged epilogue: its LDS stage would not fit two
@@ -2087,6 +2092,7 @@ __global__ void __launch_bounds__(NW * 64) mfma_gemm_dma_kernel(Problem p) {
   static_assert(WM * WN == NW && GROUPS % NW == 0 && BM % 8 == 0, "shape");
   static_assert(AM == kDenseK || AM == kConvTap, "dma kernel: dense or tap-uniform conv only");
   static_assert(S >= 2 && S <= 4 && LPW * (S - 2) < 64, "stages");
+  static_assert(!PART || (!RP && !PP), "partial sums: plain form only");
   constexpr int kStageBytes = STAGED ? NW * WTM * (WTN + 4) * 4 : 0;
   constexpr int kSmem = S * STAGE > kStageBytes ? S * STAGE : kStageBytes;
   __shared__ __attribute__((aligned(1024))) uint8_t smem[kSmem];
@@ -2326,6 +2332,14 @@ __global__ void __launch_bounds__(NW * 64) mfma_gemm_dma_kernel(Problem p) {
         for (int j = 0; j < TN; ++j) acc[i][j] += acc_odd[i][j];
     }
   } else {
+  acc_t total[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      if constexpr (PART) total[i][j] = acc_t{-0.0f, -0.0f, -0.0f, -0.0f};  // -0 + x = x
+    }
+  int left = PART ? p.k_part / BK : 0;
 #pragma unroll
   for (int st = 0; st < S - 1; ++st)
     if (st < ktiles) issue(st, st);
@@ -2381,6 +2395,24 @@ __global__ void __launch_bounds__(NW * 64) mfma_gemm_dma_kernel(Problem p) {
         }
     if constexpr (kPrio) __builtin_amdgcn_s_setprio(0);
     __builtin_amdgcn_sched_barrier(0);
+    if constexpr (PART) {
+      if (--left == 0) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int j = 0; j < TN; ++j) {
+            total[i][j] += acc[i][j];
+            acc[i][j] = acc_t{0, 0, 0, 0};
+          }
+        left = p.k_part / BK;
+      }
+    }
+  }
+  if constexpr (PART) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) acc[i][j] = total[i][j];
   }
   }
 
@@ -2590,6 +2622,7 @@ inline int ks_tile(const Problem& p, int64_t batch, int cus, int elem_bytes) {
   return tiles32 <= 2 * cus || (tiles32 <= 4 * cus && p.k * elem_bytes >= 6144) ? 2 : 0;
 }
 int launch_ks_16(Problem p, hipStream_t s, int in_dtype, int am, int tile);          // gemm_ks_16.hip
+int launch_ks_16_part(Problem p, hipStream_t s, int in_dtype, int tile);             // gemm_ks_16.hip
 int launch_ks_i8(Problem p, hipStream_t s, int mode, int out_dtype, int tile);       // gemm_ks_8.hip
 int launch_ks_f8(Problem p, hipStream_t s, int out_dtype, int tile);                 // gemm_ks_8.hip
 int launch_ks_f32(Problem p, hipStream_t s, int am, int tile);                       // gemm_ks_8.hip
@@ -2613,19 +2646,22 @@ inline int mid_tile(const Problem& p, int64_t batch, int cus, int am, int elem_b
   const int64_t tiles128 = ceil_div(p.m, 128) * ceil_div(p.n, 128);
   return tiles128 <= cus || (am == kDenseK && p.k * elem_bytes <= 1024 && 2 * tiles128 <= 3 * cus) ? 2 : 0;
 }
-template <typename Mma, typename TO, int AM>
+template <typename Mma, typename TO, int AM, bool PART = false>
 int launch_mid_tile(Problem p, hipStream_t s, int tile, const char* what) {
   dim3 grid;
   if (tile == 1) {
     grid_of<64, 64>(p, 1, grid);
-    hipLaunchKernelGGL((mfma_gemm_dma_kernel<Mma, TO, 64, 64, 4, 1, AM, 2>), grid, dim3(kThreads), 0, s, p);
+    hipLaunchKernelGGL((mfma_gemm_dma_kernel<Mma, TO, 64, 64, 4, 1, AM, 2, 4, false, false, PART>), grid, dim3(kThreads), 0,
+                       s, p);
   } else {
     grid_of<128, 64>(p, 1, grid);
-    hipLaunchKernelGGL((mfma_gemm_dma_kernel<Mma, TO, 128, 64, 4, 1, AM, 2>), grid, dim3(kThreads), 0, s, p);
+    hipLaunchKernelGGL((mfma_gemm_dma_kernel<Mma, TO, 128, 64, 4, 1, AM, 2, 4, false, false, PART>), grid,
+                       dim3(kThreads), 0, s, p);
   }
   return launch_status(what);
 }
 int launch_mid_16(Problem p, hipStream_t s, int in_dtype, int am, int tile);         // gemm_mid_16.hip
+int launch_mid_16_part(Problem p, hipStream_t s, int in_dtype, int tile);            // gemm_mid_16.hip
 int launch_mid_i8(Problem p, hipStream_t s, int mode, int out_dtype, int tile);      // gemm_mid_8.hip
 int launch_mid_f8(Problem p, hipStream_t s, int out_dtype, int tile);                // gemm_mid_8.hip
 

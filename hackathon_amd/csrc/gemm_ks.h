@@ -258,8 +258,11 @@ struct TileLoads {
 // the next round's fragments under the MFMAs of this one's while the loaders
 // refill the stage before.  (Owners that also load stall on the issue of
 // their loads behind the CU's other loads, with their LDS reads after it: a
-// K tile then took 270 clocks in place of 120.)
-template <typename Mma, typename TO, int AM, int BM, int BN, int OM, int ON, int NL, int G, int S>
+// K tile then took 270 clocks in place of 120.)  PART: the accumulators are
+// added to a total and restarted after every p.k_part of K -- the fp32
+// partials and the ordered sum of a split-K GEMM (splitk_reduce_kernel),
+// with neither in memory.
+template <typename Mma, typename TO, int AM, int BM, int BN, int OM, int ON, int NL, int G, int S, bool PART>
 __global__ void __launch_bounds__((OM * ON + NL) * 64) gemm_ordered_kernel(Problem p) {
   constexpr int BK = 128 / Mma::ES, KS = 8 / Mma::kStep;
   constexpr int TM = BM / OM / 16, TN = BN / ON / 16;
@@ -315,11 +318,15 @@ __global__ void __launch_bounds__((OM * ON + NL) * 64) gemm_ordered_kernel(Probl
   }
 
   const int row0 = wave / ON * 16 * TM, col0 = wave % ON * 16 * TN;  // this wave's piece of the tile
-  acc_t acc[TM][TN];
+  acc_t acc[TM][TN], total[TM][TN];
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
-    for (int j = 0; j < TN; ++j) acc[i][j] = acc_t{0, 0, 0, 0};
+    for (int j = 0; j < TN; ++j) {
+      acc[i][j] = acc_t{0, 0, 0, 0};
+      total[i][j] = acc_t{-0.0f, -0.0f, -0.0f, -0.0f};  // -0 + x = x
+    }
+  int left = PART ? p.k_part / BK : 0;
   vec av[2][G][KS][TM], bv[2][G][KS][TN];
   auto read_frags = [&](auto set_c, int st) {
     constexpr int SET = decltype(set_c)::value;
@@ -344,6 +351,16 @@ __global__ void __launch_bounds__((OM * ON + NL) * 64) gemm_ordered_kernel(Probl
     constexpr int SET = decltype(set_c)::value;
 #pragma unroll
     for (int q = 0; q < KS; ++q) mma_step<Mma, TM, TN>(acc, av[SET][t][q], bv[SET][t][q]);
+    if (PART && --left == 0) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          total[i][j] += acc[i][j];
+          acc[i][j] = acc_t{0, 0, 0, 0};
+        }
+      left = p.k_part / BK;
+    }
   };
   OutPiece<Mma, TO> piece[TM][TN];  // C^T accumulators: row l16, columns 4 lg + r
 #pragma unroll
@@ -383,7 +400,7 @@ __global__ void __launch_bounds__((OM * ON + NL) * 64) gemm_ordered_kernel(Probl
   for (int i = 0; i < TM; ++i)
 #pragma unroll
     for (int j = 0; j < TN; ++j)
-      if (piece[i][j].live) piece[i][j].finish(__builtin_bit_cast(float4, acc[i][j]));
+      if (piece[i][j].live) piece[i][j].finish(__builtin_bit_cast(float4, PART ? total[i][j] : acc[i][j]));
 }
 
 // Tiles of launch_ordered_*: 1 = 16 x 32 (one workgroup per CU: the rule
@@ -395,16 +412,17 @@ __global__ void __launch_bounds__((OM * ON + NL) * 64) gemm_ordered_kernel(Probl
 // 1 x 7 x 7 x 512 6.3 / 6.9, 8 x 14 x 14 x 256 8.4 / 9.4, 16 x 7 x 7 x 512
 // 14.5 / 15.5 -- and 128 x 128 tiles 8.6, 21.8, 21.9, 24.7, 35.1; 49.8, 26.5,
 // 46.1.
-template <typename Mma, typename TO, int AM>
+template <typename Mma, typename TO, int AM, bool PART = false>
 int launch_ordered_tile(Problem p, hipStream_t s, int tile, const char* what) {
   dim3 grid;
   if (tile == 1) {
     constexpr int NL = AM == kConvTap ? 6 : 4;
     grid_of<16, 32>(p, 1, grid);
-    hipLaunchKernelGGL((gemm_ordered_kernel<Mma, TO, AM, 16, 32, 1, 2, NL, NL, 3>), grid, dim3(64 * (2 + NL)), 0, s, p);
+    hipLaunchKernelGGL((gemm_ordered_kernel<Mma, TO, AM, 16, 32, 1, 2, NL, NL, 3, PART>), grid, dim3(64 * (2 + NL)), 0,
+                       s, p);
   } else {
     grid_of<32, 32>(p, 1, grid);
-    hipLaunchKernelGGL((gemm_ordered_kernel<Mma, TO, AM, 32, 32, 2, 2, 4, 2, 3>), grid, dim3(512), 0, s, p);
+    hipLaunchKernelGGL((gemm_ordered_kernel<Mma, TO, AM, 32, 32, 2, 2, 4, 2, 3, PART>), grid, dim3(512), 0, s, p);
   }
   return launch_status(what);
 }

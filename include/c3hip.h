@@ -712,14 +712,25 @@ int c3h_gemm_splitk_reduce(const c3h_splitk_args* a, void* stream);
  * (batch 1) cut along K into `splits` partial GEMMs of K/splits each, fp32
  * partials written to `workspace` ([splits][m][n], splits*m*n*4 bytes,
  * 16-byte aligned), then the ordered reduce of c3h_gemm_splitk_reduce with
- * a's epilogue into a->out: the two launches the compiled engine issues for
- * a bf16 GEMM with too few output tiles to fill the chip (the ResNet-18 224
- * classifier; fused_gemm_epilogue_f32, R:606-633), for
- * callers outside the compiled engine.  k must be a multiple of splits
+ * a's epilogue into a->out.  16-bit outputs of few tiles whose K/splits is a
+ * multiple of 64 form the same partials and the same ordered sum in registers
+ * instead, in one launch, and leave the workspace alone.  The compiled engine
+ * runs every 16-bit GEMM with too few output tiles to fill the chip this way
+ * (the ResNet-18 224 classifier, the Linears of a short prompt;
+ * fused_gemm_epilogue_f32, R:606-633).  k must be a multiple of splits
  * (1 <= splits <= 64; 16-bit inputs: K/splits a multiple of 8); the
  * workspace is written before it is read.  Deterministic for a given split. */
 int c3h_gemm_splitk(const c3h_gemm_args* a, int32_t splits, void* workspace, size_t workspace_bytes,
                     void* stream);
+/* The same from one argument struct, for program ops. */
+typedef struct {
+  c3h_gemm_args gemm;
+  void* workspace;
+  int64_t workspace_bytes;
+  int32_t splits;
+  int32_t pad_;
+} c3h_gemm_splitk_args;
+int c3h_gemm_splitk_launch(const c3h_gemm_splitk_args* a, void* stream);
 
 /* c3h_gemm_splitk with no workspace and no allocation: the fp32 partials go
  * to a static 32 MiB device array of the library (one per GPU, held until
@@ -866,7 +877,8 @@ enum c3h_op_kind {
   C3H_OP_GEMM_W4A16 = 37,
   C3H_OP_ARGMAX_FINISH = 38,
   C3H_OP_NONFINITE = 39,
-  C3H_OP_FLASH_F32 = 40
+  C3H_OP_FLASH_F32 = 40,
+  C3H_OP_GEMM_SPLITK = 41
 };
 
 typedef struct {
@@ -901,7 +913,7 @@ int c3h_graph_destroy(void* graph_exec);
  * c3h_quantize_args, c3h_qgemm_args, c3h_dequantize_args, c3h_op,
  * c3h_pack_args, c3h_conv_pool_args, c3h_fp8_quant_args, c3h_fp8_gemm_args,
  * c3h_splitk_args, c3h_mxfp4_quant_args, c3h_w4a16_gemm_args,
- * c3h_argmax_finish_args, c3h_nonfinite_args.
+ * c3h_argmax_finish_args, c3h_nonfinite_args, c3h_gemm_splitk_args.
  * Returns the number of sizes available (host-only; needs no GPU). */
 int32_t c3h_abi_sizes(int64_t* out, int32_t capacity);
 

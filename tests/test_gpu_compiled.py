@@ -314,6 +314,22 @@ def test_compiled_16bit_splitk_classifier(gpu, batch):
     assert diff <= 2e-2 * scale
 
 
+@pytest.mark.parametrize("policy", ["fp16", "bf16"])
+@pytest.mark.parametrize("batch,seq", [(1, 16), (3, 67)])
+def test_compiled_decoder_of_few_rows_keeps_the_split_sums(gpu, policy, batch, seq):
+    """Every Linear of a short prompt sums K in partials that are added in order.  Logits with the partials in
+    registers equal, bit for bit, those of the batched partial GEMMs and the reduce (C3H_DISABLE_DMA)."""
+    from hackathon_amd import models
+    from switches import with_switch
+
+    m = models.build_decoder(precision=policy, name="decoder", batch=batch, seq=seq, d_model=256, heads=4, ffn=1024,
+                             layers=2, vocab=1000)
+    run = lambda: _logits(_compiled(m, policy)[1], m.inputs)["logits"]
+    got, want = run(), with_switch("C3H_DISABLE_DMA", "1", run)
+    assert want.view(np.uint8).any()
+    np.testing.assert_array_equal(got.view(np.uint8), want.view(np.uint8))
+
+
 def test_compiled_gather_out_of_range_ids_raise(gpu):
     """Token ids outside the vocabulary make the compiled program raise
     IndexError after the run (np.take's behaviour in the oracle) instead of

@@ -1439,6 +1439,47 @@ def test_gemm_splitk_one_call_equals_two_launches(gpu, kind, m, n, k, splits):
     assert rc != 0 and "workspace" in _lib.last_error()
 
 
+@pytest.mark.parametrize("kind", ["fp16", "bf16"])
+@pytest.mark.parametrize("m,n,k,splits,form", [
+    (1, 512, 512, 8, "relu"), (200, 500, 2048, 32, "gelu"), (7, 33, 192, 3, "scaled"),      # 16 x 32 tiles
+    (200, 1536, 512, 8, "program"), (333, 513, 2048, 16, "relu"), (700, 700, 128, 2, "scaled"),  # 32 x 32
+    (333, 2048, 512, 4, "gelu"), (1000, 1030, 640, 5, "scaled"), (1500, 2056, 512, 2, "relu")])  # 64-column tiles
+def test_gemm_splitk_in_one_launch_keeps_the_bits(gpu, kind, m, n, k, splits, form):
+    """The partial sums of a 16-bit split-K GEMM kept in registers (small and 64-column tiles) and the two
+    launches over the workspace (C3H_DISABLE_SMALLTILE) give the same bits, in both output types; with the
+    output over the A operand c3h_gemm_splitk keeps to the two launches, which read all of A first."""
+    from hackathon_amd import _lib
+    from hackathon_amd.c35 import engine as E
+    from hackathon_amd.device import DeviceArray
+
+    rng = np.random.default_rng(m + n + k)
+    a, b, res = (_bits(rng.standard_normal(s, dtype=np.float32), kind)[0] for s in ((m, k), (n, k), (m, n)))
+    bias, bd, rd = _dev(rng.standard_normal(n, dtype=np.float32)), _dev(b), _dev(res)
+    prog = [(_lib.EW_MUL, 0, 2, 0.0), (_lib.EW_ADD, 1, 0, 0.0)]
+    kw = {"relu": dict(act=1), "gelu": dict(act=2, imm=[math.sqrt(2.0), 1.0, 0.5]), "scaled": dict(alpha=0.7, beta=0.3),
+          "program": dict(program=prog, imm=[0.25])}[form]
+
+    def run(f32=False, over_a=False):
+        ad = _dev(a)
+        out = ad if over_a else DeviceArray.from_host(np.zeros((m, n), np.float32 if f32 else a.dtype))
+        s = _lib.GemmSplitKArgs()
+        ws = DeviceArray.empty((splits, m, n), np.float32)
+        s.workspace, s.workspace_bytes, s.splits = ws.ptr, ws.nbytes, splits
+        g = s.gemm
+        g.a, g.b, g.out, g.m, g.n, g.k, g.lda, g.ldb, g.ldo, g.batch = ad.ptr, bd.ptr, out.ptr, m, n, k, k, k, n, 1
+        g.trans_b, g.in_dtype, g.out_dtype = 1, bd.code, _lib.F32 if f32 else bd.code
+        g.epi = E.epilogue(bias=bias, bias_mode=2, residual=None if f32 else rd, **kw)
+        _lib.launch(s)
+        return out.get().reshape(-1)[: m * n].view(np.uint8)
+
+    for f32 in (False, True):
+        got, want = run(f32), switches.with_switch("C3H_DISABLE_SMALLTILE", "1", lambda: run(f32))
+        assert want.any()
+        np.testing.assert_array_equal(got, want)
+    if n <= k:
+        np.testing.assert_array_equal(run(over_a=True), run())
+
+
 @pytest.mark.parametrize("rows,cols,dt,res", [(16 * 1024, 768, "bf16", False), (37, 512, "fp16", True),
                                               (5, 1024, "fp32", True), (9, 24, "bf16", False),
                                               (16 * 1024, 768, "bf16", True)])
