@@ -1576,9 +1576,7 @@ class CompiledPlan:
         one-sequence decoder's 283)."""
         if getattr(self, "_errflag", None) is None:
             self._errflag = self._keep(PinnedArray((1,), np.int32))
-            a = _lib.FillArgs()  # by a kernel on the null stream: finished before the plan's stream runs
-            a.out, a.count, a.dtype, a.value = self._errflag.ptr, 1, _lib.I32, 0.0
-            _lib.launch(a, None)
+            self._errflag.array[0] = 0  # by the host: a launch would not be ordered before the plan's stream
         return self._errflag
 
     @property

@@ -102,11 +102,15 @@ class _RecordingLib:
     def __init__(self):
         self.addr = 1 << 24
         self.calls = collections.Counter()
+        self.host = []
 
     def __getattr__(self, name):
         def fn(*args):
             self.calls[name] += 1
-            if name in ("c3h_malloc", "c3h_host_alloc"):
+            if name == "c3h_host_alloc":  # memory the host writes: real, and not zero
+                self.host.append(C.create_string_buffer(b"\xa5" * int(args[1]), int(args[1])))
+                args[0]._obj.value = C.addressof(self.host[-1])
+            elif name == "c3h_malloc":
                 args[0]._obj.value = self.addr
                 self.addr += (int(args[1]) + 4095) // 4096 * 4096 + 4096
             elif name in ("c3h_stream_create", "c3h_event_create"):
@@ -163,6 +167,15 @@ def test_compiled_lowering_launch_groups(fake_lib, name, policy, expect):
         if meta["kind"].split(":")[0] in ("conv", "gemm", "qgemm", "flash"):
             assert meta["flops"] > 0
         assert meta["bytes"] > 0
+
+
+def test_compiled_gather_flag_is_cleared_by_the_host(fake_lib):
+    """The pinned flag is zero once the program is built, with no launch for it: the plan's stream does not wait
+    for other streams, so a fill launched elsewhere could erase the flag of a real out-of-range index."""
+    _, prog = _lower("decoder_fp16", "fp16")
+    assert int(prog.error_flag.array[0]) == 0
+    assert fake_lib.calls["c3h_fill"] == 0
+    prog.check_errors()
 
 
 @pytest.mark.parametrize("name,policy", [("resnet18_224", "bf16"), ("decoder_fp16", "fp16"), ("decoder_w8a8", "w8a8")])
