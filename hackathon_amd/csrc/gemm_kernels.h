@@ -728,6 +728,32 @@ __device__ __forceinline__ void mma_step(Acc (&acc)[TM][TN], const Vec (&av)[TM]
   }
 }
 
+// The same into CH chains of accumulators: element e of an fp32 chunk goes to
+// chain e % CH.
+template <typename Mma, int TM, int TN, int CH, typename Acc, typename Vec>
+__device__ __forceinline__ void mma_chains(Acc (&acc)[CH][TM][TN], const Vec (&av)[TM], const Vec (&bv)[TN]) {
+  if constexpr (CH == 1) {
+    mma_step<Mma, TM, TN>(acc[0], av, bv);
+  } else {
+    static_assert(std::is_same<Mma, MmaF32>::value, "one chain per output but in fp32");
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+          acc[e % CH][i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bv[j][e], av[i][e], acc[e % CH][i][j], 0, 0, 0);
+  }
+}
+// An output's chains, added pairwise.
+template <int TM, int TN, int CH, typename Acc>
+__device__ __forceinline__ Acc chain_sum(const Acc (&acc)[CH][TM][TN], int i, int j) {
+  static_assert(CH == 1 || CH == 2 || CH == 4, "pairs");
+  if constexpr (CH == 1) return acc[0][i][j];
+  else if constexpr (CH == 2) return acc[0][i][j] + acc[1][i][j];
+  else return (acc[0][i][j] + acc[1][i][j]) + (acc[2][i][j] + acc[3][i][j]);
+}
+
 // MFMA operand of tile row `r` (row base `row`, XOR-swizzled 16-byte chunks)
 // for the K step starting at chunk ks.
 template <typename Mma>

@@ -457,11 +457,18 @@ __global__ void __launch_bounds__(KW * 64) gemm_ks_kernel(Problem p) {
   OutPiece<Mma, TO> piece;
   piece.load(m0 + o_row, n0 + o_col, tid < BM * NC);
 
-  acc_t acc[TM][TN];
+  // fp32: the four MFMAs of a 16-byte chunk sum apart.  One chain per wave
+  // rounded K / KW terms in a row, which lost precision to the split-K this
+  // kernel replaces (error against 64 bits, split-K / one chain / four, 1e-7:
+  // 256 x 512 x 784 in 14 splits 1.54 / 1.87 / 1.14, 16 x 512 x 2048 in 64 1.79 / 2.88 / 1.59).
+  constexpr int CH = std::is_same<Mma, MmaF32>::value ? 4 : 1;
+  acc_t acc[CH][TM][TN];
 #pragma unroll
-  for (int i = 0; i < TM; ++i)
+  for (int c = 0; c < CH; ++c)
 #pragma unroll
-    for (int j = 0; j < TN; ++j) acc[i][j] = acc_t{0, 0, 0, 0};
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) acc[c][i][j] = acc_t{0, 0, 0, 0};
 
   // This wave's K tiles: wave, wave + KW, ...
   const int nkt = static_cast<int>(ceil_div(p.k, BK));
@@ -490,7 +497,7 @@ __global__ void __launch_bounds__(KW * 64) gemm_ks_kernel(Problem p) {
       issue(wave + KW * (r + S), r & 1);
     }
 #pragma unroll
-    for (int q = 0; q < KS; ++q) mma_step<Mma, TM, TN>(acc, av[q], bv[q]);
+    for (int q = 0; q < KS; ++q) mma_chains<Mma, TM, TN>(acc, av[q], bv[q]);
   }
 
   // The waves' partial tiles, summed in wave order.
@@ -502,7 +509,7 @@ __global__ void __launch_bounds__(KW * 64) gemm_ks_kernel(Problem p) {
 #pragma unroll
     for (int j = 0; j < TN; ++j)
       *reinterpret_cast<float4*>(part + (16 * i + l16) * SS + 16 * j + 4 * lg) =
-          __builtin_bit_cast(float4, acc[i][j]);  // C^T accumulators: row l16, columns 4 lg + r
+          __builtin_bit_cast(float4, chain_sum<TM, TN>(acc, i, j));  // C^T accumulators: row l16, columns 4 lg + r
   __syncthreads();
   if (!piece.live) return;
   const float* src = stage + o_row * SS + o_col;

@@ -1439,6 +1439,36 @@ def test_gemm_splitk_one_call_equals_two_launches(gpu, kind, m, n, k, splits):
     assert rc != 0 and "workspace" in _lib.last_error()
 
 
+@pytest.mark.parametrize("m,n,k,splits", [(256, 512, 784, 14), (256, 256, 512, 16), (200, 512, 2048, 16),
+                                          (16, 512, 2048, 64), (333, 512, 2048, 8), (1000, 512, 2048, 4)])
+def test_small_fp32_gemm_is_no_less_exact_than_split_k(gpu, m, n, k, splits):
+    """fp32 GEMMs of few output tiles round in chains no longer than the K splits of c3h_gemm_splitk at the same
+    size (`splits` gives every CU at most two 64 x 64 tiles): 2-norm error against float64 no larger.  Rounding
+    errors add as in a random walk, so over these outputs the two norms are good to well under the 25 % between
+    them (one chain per wave was 10 to 50 % above split-K, four are 25 to 50 % below)."""
+    from hackathon_amd import _lib
+    from hackathon_amd.c35 import engine as E
+    from hackathon_amd.device import DeviceArray
+
+    rng = np.random.default_rng(k + m)
+    a = rng.standard_normal((m, k), dtype=np.float32)
+    b = (rng.standard_normal((n, k)) / math.sqrt(k)).astype(np.float32)
+    ad, bd = _dev(a), _dev(b)
+    exact = a.astype(np.float64) @ b.T.astype(np.float64)
+    outs = [DeviceArray.empty((m, n), np.float32) for _ in range(2)]
+    g = _lib.GemmArgs()
+    g.a, g.b, g.m, g.n, g.k, g.lda, g.ldb, g.ldo, g.batch = ad.ptr, bd.ptr, m, n, k, k, k, n, 1
+    g.trans_b, g.in_dtype, g.out_dtype = 1, _lib.F32, _lib.F32
+    g.epi = E.epilogue()
+    g.out = outs[0].ptr
+    _lib.launch(g)
+    g.out = outs[1].ptr
+    E.gemm_splitk(g, splits, DeviceArray.empty((splits, m, n), np.float32))
+    got, want = (np.linalg.norm(o.get() - exact) / np.linalg.norm(exact) for o in outs)
+    print("error %.3e, split-K %.3e" % (got, want))
+    assert 0.0 < got <= want
+
+
 @pytest.mark.parametrize("kind", ["fp16", "bf16"])
 @pytest.mark.parametrize("m,n,k,splits,form", [
     (1, 512, 512, 8, "relu"), (200, 500, 2048, 32, "gelu"), (7, 33, 192, 3, "scaled"),      # 16 x 32 tiles
