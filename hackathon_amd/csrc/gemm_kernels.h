@@ -708,49 +708,37 @@ struct MmaF32 {
 };
 
 // One K step of a wave tile: acc[i][j] += bv[j] x av[i] (operands swapped,
-// C^T: see epilogue_direct).  fp32 walks the four MFMAs of a chunk outermost,
-// so that consecutive MFMAs go to different accumulators.
+// C^T: see epilogue_direct).
 template <typename Mma, int TM, int TN, typename Acc, typename Vec>
 __device__ __forceinline__ void mma_step(Acc (&acc)[TM][TN], const Vec (&av)[TM], const Vec (&bv)[TN]) {
-  if constexpr (std::is_same<Mma, MmaF32>::value) {
 #pragma unroll
-    for (int e = 0; e < 4; ++e)
+  for (int i = 0; i < TM; ++i)
 #pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bv[j][e], av[i][e], acc[i][j], 0, 0, 0);
-  } else {
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j) acc[i][j] = Mma::mma(bv[j], av[i], acc[i][j]);
-  }
+    for (int j = 0; j < TN; ++j) acc[i][j] = Mma::mma(bv[j], av[i], acc[i][j]);
 }
-
-// The same into CH chains of accumulators: element e of an fp32 chunk goes to
-// chain e % CH.
+// The same into CH chains of accumulators: one, but in fp32 four, one for each
+// element of a 16-byte chunk (walked outermost, so that consecutive MFMAs go
+// to different accumulators).
 template <typename Mma, int TM, int TN, int CH, typename Acc, typename Vec>
 __device__ __forceinline__ void mma_chains(Acc (&acc)[CH][TM][TN], const Vec (&av)[TM], const Vec (&bv)[TN]) {
-  if constexpr (CH == 1) {
+  if constexpr (!std::is_same<Mma, MmaF32>::value) {
+    static_assert(CH == 1, "one chain");
     mma_step<Mma, TM, TN>(acc[0], av, bv);
   } else {
-    static_assert(std::is_same<Mma, MmaF32>::value, "one chain per output but in fp32");
+    static_assert(CH == 4, "a chain per element");
 #pragma unroll
     for (int e = 0; e < 4; ++e)
 #pragma unroll
       for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j)
-          acc[e % CH][i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bv[j][e], av[i][e], acc[e % CH][i][j], 0, 0, 0);
+          acc[e][i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bv[j][e], av[i][e], acc[e][i][j], 0, 0, 0);
   }
 }
 // An output's chains, added pairwise.
 template <int TM, int TN, int CH, typename Acc>
 __device__ __forceinline__ Acc chain_sum(const Acc (&acc)[CH][TM][TN], int i, int j) {
-  static_assert(CH == 1 || CH == 2 || CH == 4, "pairs");
   if constexpr (CH == 1) return acc[0][i][j];
-  else if constexpr (CH == 2) return acc[0][i][j] + acc[1][i][j];
   else return (acc[0][i][j] + acc[1][i][j]) + (acc[2][i][j] + acc[3][i][j]);
 }
 
@@ -2284,13 +2272,16 @@ __global__ void __launch_bounds__(NW * 64) mfma_gemm_dma_kernel(Problem p) {
     constexpr int N_DSR = KS * (TM + TN) * (Mma::kStep == 8 ? 2 : 1);
     constexpr int PER = N_MFMA / N_DSR;
     vec av[2][KS][TM], bv[2][KS][TN];
-    // fp32: the odd K steps sum apart, so a long K rounds in two chains of
-    // half its length.
-    acc_t acc_odd[TM][TN];
+    // fp32: the four MFMAs of a 16-byte chunk sum apart, so a long K rounds in
+    // four chains of a quarter of its length.
+    constexpr int CH = std::is_same<Mma, MmaF32>::value ? 4 : 1;
+    acc_t chains[CH][TM][TN];
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
+    for (int c = 0; c < CH; ++c)
 #pragma unroll
-      for (int j = 0; j < TN; ++j) acc_odd[i][j] = acc_t{0, 0, 0, 0};
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) chains[c][i][j] = acc_t{0, 0, 0, 0};
     auto read_frags = [&](auto set_c, int stage) {
       constexpr int SET = decltype(set_c)::value;
       const uint8_t* As = smem + stage * STAGE;
@@ -2335,10 +2326,7 @@ __global__ void __launch_bounds__(NW * 64) mfma_gemm_dma_kernel(Problem p) {
       // between every PER MFMAs of tile kt.
       read_frags(std::integral_constant<int, SET ^ 1>{}, static_cast<int>((kt + 1) % S));
 #pragma unroll
-      for (int q = 0; q < KS; ++q) {
-        if constexpr (std::is_same<Mma, MmaF32>::value) mma_step<Mma, TM, TN>(q ? acc_odd : acc, av[SET][q], bv[SET][q]);
-        else mma_step<Mma, TM, TN>(acc, av[SET][q], bv[SET][q]);
-      }
+      for (int q = 0; q < KS; ++q) mma_chains<Mma, TM, TN>(chains, av[SET][q], bv[SET][q]);
 #pragma unroll
       for (int g = 0; g < N_DSR; ++g) {
         __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);    // one LDS read
@@ -2351,12 +2339,10 @@ __global__ void __launch_bounds__(NW * 64) mfma_gemm_dma_kernel(Problem p) {
       body(std::integral_constant<int, 0>{}, kt);
       if (kt + 1 < ktiles) body(std::integral_constant<int, 1>{}, kt + 1);
     }
-    if constexpr (std::is_same<Mma, MmaF32>::value) {
 #pragma unroll
-      for (int i = 0; i < TM; ++i)
+    for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int j = 0; j < TN; ++j) acc[i][j] += acc_odd[i][j];
-    }
+      for (int j = 0; j < TN; ++j) acc[i][j] = chain_sum<TM, TN>(chains, i, j);
   } else {
   acc_t total[TM][TN];
 #pragma unroll

@@ -1440,7 +1440,8 @@ def test_gemm_splitk_one_call_equals_two_launches(gpu, kind, m, n, k, splits):
 
 
 @pytest.mark.parametrize("m,n,k,splits", [(256, 512, 784, 14), (256, 256, 512, 16), (200, 512, 2048, 16),
-                                          (16, 512, 2048, 64), (333, 512, 2048, 8), (1000, 512, 2048, 4)])
+                                          (16, 512, 2048, 64), (333, 512, 2048, 8), (1000, 512, 2048, 4),
+                                          (700, 768, 768, 3), (700, 768, 3072, 3)])
 def test_small_fp32_gemm_is_no_less_exact_than_split_k(gpu, m, n, k, splits):
     """fp32 GEMMs of few output tiles round in chains no longer than the K splits of c3h_gemm_splitk at the same
     size (`splits` gives every CU at most two 64 x 64 tiles): 2-norm error against float64 no larger.  Rounding
