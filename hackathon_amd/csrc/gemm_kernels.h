@@ -2825,19 +2825,26 @@ int launch_w4_tile(Problem p, hipStream_t s) {
   hipLaunchKernelGGL((mfma_gemm_kernel<MmaF16, TO, BM, BN, WM, WN, kDenseK, true, true>), grid, dim3(kThreads), 0, s, p);
   return launch_status("gemm_w4a16");
 }
-// 64 x 64 tiles up to four per CU, then 128 x 64 up to 1.5 tiles of 128 x 128
-// per CU, or past two where K is at most 1024 (the epilogue's share is large);
-// measured (M x N x K, us, 128 x 128 / 64 x 64 / 128 x 64): 200 x 512 x 2048
-// 34.4 / 17.4 / 23.5, 3000 x 512 x 2048 37.6 / 24.4 / 26.9, 3000 x 2048 x 512
-// 22.8 / 20.3 / 18.7, 6000 x 768 x 3072 63.1 / 66.5 / 55.2, 6000 x 2304 x 768
-// 48.3 / 49.0 / 44.9, 16384 x 512 x 2048 49.9 / 64.2 / 58.6.  Every tile sums
-// K in the same order.
+// 64 x 64 tiles up to three per CU, then 128 x 64 up to 1.5 tiles of 128 x 128
+// per CU and, where K is at most 1024, between 2 and 2.5 of them: 128 x 128
+// runs two blocks per CU, and its last round would be nearly empty.  From
+// there on 128 x 128, which widens each weight for twice the rows.  Measured (M
+// x N x K, us, 128 x 128 / 128 x 64 / 64 x 64): 333 x 512 x 2048 27.1 / 20.2 /
+// 16.3, 4000 x 768 x 3072 (756 tiles of 64 x 64) 44.0 / 40.2 / 38.0, 2048 x
+// 2048 x 512 (1024) 11.3 / 10.9 / 11.7, 8000 x 512 x 2048 (1000) 31.4 / 29.2 /
+// 32.4; 3000 x 2048 x 512 (384 tiles of 128 x 128) 17.0 / 14.4 / 16.7, 8000 x
+// 1000 x 512 (504) 18.0 / 20.4 / 19.7, 6000 x 1536 x 512 (564) 24.2 / 21.0 /
+// 23.2, 13000 x 768 x 768 (612) 29.7 / 27.4 / 32.6, 7000 x 1536 x 512 (660)
+// 23.0 / 23.8 / 26.0, 15000 x 768 x 768 (708) 30.0 / 32.0 / 37.7, 16384 x 1536
+// x 512 (1536) 43.1 / 46.3 / 58.0, 16384 x 8192 x 512 (8192) 189 / 210 / 260.
+// Every tile sums K in the same order.
 template <typename TO>
 int launch_w4(Problem p, hipStream_t s) {
   const int64_t cus = device_cus(), tiles128 = ceil_div(p.m, 128) * ceil_div(p.n, 128);
-  if (ceil_div(p.m, 64) * ceil_div(p.n, 64) <= 4 * cus) return launch_w4_tile<TO, 64, 64, 4, 1>(p, s);
+  if (ceil_div(p.m, 64) * ceil_div(p.n, 64) <= 3 * cus) return launch_w4_tile<TO, 64, 64, 4, 1>(p, s);
   if (p.n <= 64) return launch_w4_tile<TO, 256, 64, 4, 1>(p, s);
-  if (2 * tiles128 <= 3 * cus || (p.k <= 1024 && tiles128 > 2 * cus)) return launch_w4_tile<TO, 128, 64, 4, 1>(p, s);
+  if (2 * tiles128 <= 3 * cus || (p.k <= 1024 && tiles128 > 2 * cus && 2 * tiles128 <= 5 * cus))
+    return launch_w4_tile<TO, 128, 64, 4, 1>(p, s);
   return launch_w4_tile<TO, 128, 128, 2, 2>(p, s);
 }
 
