@@ -2614,16 +2614,22 @@ inline int device_cus() {
 }
 
 // Whether a small-output kernel takes this GEMM or tap-uniform conv, and on
-// which tile (gemm_ks.h; 0 = no, 1 = 16 x 32, 2 = 32 x 32): outputs of at
-// most one 16 x 32 tile, or two 32 x 32 tiles, per CU -- four where K is at
-// least 6 KB per row, which the shared tiles walk at 0.5 us per 128 bytes.
-// Measured on 256 CUs against the best shared-tile kernel (M x N x K, us):
-// 333 x 512 x 2048 5.5 / 12.2, 200 x 2304 x 768 (504 tiles of 32 x 32) 5.2 /
-// 7.4, 1000 x 512 x 2048 (512) 8.8 / 12.7; past the line 333 x 2048 x 512
-// (704) 7.7 / 6.3 and 2048 x 512 x 2048 (1024) 15.9 / 12.5, but 1000 x 768 x
-// 3072 (768) 15.9 / 26.3.  16 x 32 over 32 x 32 where both fit: 200 x 512 x
-// 2048 4.5 / 5.3, in fp32 (MFMA-bound: twice the CUs) 8.7 / 13.2.  Row-major
+// which tile (gemm_ks.h; 0 = no, 1 = 16 x 32, 2 = 32 x 32): outputs of at most
+// one 16 x 32 tile, or two 32 x 32 tiles, per CU -- four where K is at least 6
+// KB per row, which the shared tiles walk at 0.5 us per 128 bytes. Row-major
 // outputs without the row_max side output only.
+//
+// Measured on 256 CUs against the best shared-tile kernel (M x N x K, us),
+// 16-bit: 333 x 512 x 2048 5.5 / 12.2, 200 x 2304 x 768 (504 tiles of 32 x 32)
+// 5.2 / 7.4, 1000 x 512 x 2048 (512) 8.8 / 12.7; past the line 333 x 2048 x
+// 512 (704) 7.7 / 6.3 and 2048 x 512 x 2048 (1024) 15.9 / 12.5, but 1000 x 768
+// x 3072 (768) 15.9 / 26.3. The deep-K line in the other types: fp32 1500 x
+// 512 x 2048 (752) 33.7 / 40.9, 2048 x 384 x 1536 (768) 26.7 / 32.0, 2048 x
+// 512 x 2048 (1024) 41.6 / 41.5 (past it 1000 x 1536 x 512 (1536) 23.4 /
+// 21.2); int8 1000 x 768 x 6144 (768) 17.6 / 27.1, 2048 x 512 x 6144 (1024)
+// 22.6 / 26.0; E4M3 17.4 / 26.2 and 19.8 / 26.9. 16 x 32 over 32 x 32 where
+// both fit: 200 x 512 x 2048 4.5 / 5.3, in fp32 (MFMA-bound: twice the CUs)
+// 9.0 / 13.3.
 inline int ks_tile(const Problem& p, int64_t batch, int cus, int elem_bytes) {
   if (batch != 1 || p.out_nchw || p.epi.row_max != nullptr || switches().disable_dma ||
       switches().disable_smalltile || p.a_bytes <= 0 || p.b_bytes <= 0 || p.a_bytes >= (int64_t{1} << 31) ||
@@ -2639,24 +2645,32 @@ int launch_ks_i8(Problem p, hipStream_t s, int mode, int out_dtype, int tile);  
 int launch_ks_f8(Problem p, hipStream_t s, int out_dtype, int tile);                 // gemm_ks_8.hip
 int launch_ks_f32(Problem p, hipStream_t s, int am, int tile);                       // gemm_ks_8.hip
 
-// Whether the four-wave DMA kernel takes this GEMM or conv on a 64-column
-// tile (0 = no, 1 = 64 x 64, 2 = 128 x 64): outputs whose 128 x 128 tiles
-// leave CUs idle or alone with one block, whose DMA wait, LDS reads and MFMAs
-// then follow one another unhidden (0.7 us per K tile at any stage count).
-// 64 x 64 up to two tiles per CU, 128 x 64 up to one 128 x 128 tile per CU --
-// and, for dense GEMMs of at most 1 KB of K per row, whose blocks are mostly
-// prologue and epilogue, up to 1.5.  Measured (bf16, M x N x K, us, 128 x 128
-// / 64 x 64 / 128 x 64): 700 x 2048 x 512 13.2 / 7.3 / 8.9, 3000 x 512 x 2048
-// 28.2 / 19.7 / 23.2, 8192 x 512 x 2048 27.8 / 28.8 / 24.9, 3000 x 2048 x 512
-// (384 tiles of 128 x 128) 18.2 / 16.6 / 13.7, 16384 x 512 x 512 (512) 14.6 /
-// 24.1 / 19.5; 3x3 convs of 128 channels 28 x 28: batch 20 16.1 / 11.4 /
-// 12.3, 37 (227 tiles) 16.9 / 16.5 / 14.5, 64 (392) 20.8 / 26.1 / 29.4.  The
-// K order is that of the other tiles: bit-identical results.
-inline int mid_tile(const Problem& p, int64_t batch, int cus, int am, int elem_bytes) {
+// Whether the four-wave DMA kernel takes this GEMM or conv on a 64-column tile
+// (0 = no, 1 = 64 x 64, 2 = 128 x 64): outputs whose 128 x 128 tiles leave CUs
+// idle or alone with one block, whose DMA wait, LDS reads and MFMAs then
+// follow one another unhidden (0.7 us per K tile at any stage count). 64 x 64
+// up to two tiles per CU, 128 x 64 up to one 128 x 128 tile per CU -- and, for
+// dense GEMMs of at most short_k bytes of K per row, whose blocks are mostly
+// prologue and epilogue, up to 1.5. short_k is 1 KB, but half of that for
+// int8, whose K loop is the cheapest part on the large tile. The K order is
+// that of the other tiles: bit-identical results.
+//
+// Measured (M x N x K, us, 128 x 128 / 64 x 64 / 128 x 64). bf16: 700 x 2048 x
+// 512 13.2 / 7.3 / 8.9, 3000 x 512 x 2048 28.2 / 19.7 / 23.2, 8192 x 512 x
+// 2048 27.8 / 28.8 / 24.9, 3000 x 2048 x 512 (384 tiles of 128 x 128) 18.2 /
+// 16.6 / 13.7, 16384 x 512 x 512 (512) 14.6 / 24.1 / 19.5; 3x3 convs of 128
+// channels 28 x 28: batch 20 16.1 / 11.4 / 12.3, 37 (227 tiles) 16.9 / 16.5 /
+// 14.5, 64 (392) 20.8 / 26.1 / 29.4. int8, then E4M3: 1000 x 3072 x 768 12.4 /
+// 9.9 / 9.1 and 10.7 / 8.1 / 7.9, 2048 x 768 x 3072 18.7 / 11.6 / 14.2 and
+// 18.8 / 11.5 / 14.1, 5000 x 768 x 3072 (240 tiles) 21.9 / 23.8 / 20.4 and
+// 21.6 / 21.7 / 19.6, 2048 x 2304 x 768 (288) 10.5 / 13.2 / 11.1 and 10.6 /
+// 12.5 / 10.1, 7000 x 768 x 768 (330) 11.9 / 14.4 / 13.1 and 10.9 / 12.2 /
+// 10.9, 3000 x 2048 x 512 (384) 14.3 / 14.0 / 11.4 and 12.0 / 11.2 / 9.8.
+inline int mid_tile(const Problem& p, int64_t batch, int cus, int am, int elem_bytes, int short_k = 1024) {
   if (switches().disable_smalltile || !dma_eligible(p, batch, am)) return 0;
   if (ceil_div(p.m, 64) * ceil_div(p.n, 64) <= 2 * cus) return 1;
   const int64_t tiles128 = ceil_div(p.m, 128) * ceil_div(p.n, 128);
-  return tiles128 <= cus || (am == kDenseK && p.k * elem_bytes <= 1024 && 2 * tiles128 <= 3 * cus) ? 2 : 0;
+  return tiles128 <= cus || (am == kDenseK && p.k * elem_bytes <= short_k && 2 * tiles128 <= 3 * cus) ? 2 : 0;
 }
 template <typename Mma, typename TO, int AM, bool PART = false>
 int launch_mid_tile(Problem p, hipStream_t s, int tile, const char* what) {
