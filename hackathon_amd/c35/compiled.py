@@ -1659,8 +1659,10 @@ class CompiledPlan:
               and q.shape[-1] == 64 and div is not None and div != 0.0
               and len(q.shape) == 4 and len(kt.shape) == 4 and q.shape[:2] == kt.shape[:2])
         mask = self._flash_mask(node.inputs[3], q.shape[2], kt.shape[3]) if ok else None
-        if mask is None:
+        if mask is None or (self.keep_values and self.act_dtype == np.float32):
+            # (keep_values under fp32: the probabilities beside the one launch, for read_value)
             self._attention_scores_materialized(node)
+        if mask is None:
             return
         self.__dict__.setdefault("_pending_attn", {})[node.outputs[0]] = (node, mask)
 

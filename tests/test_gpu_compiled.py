@@ -346,3 +346,25 @@ def test_compiled_gather_out_of_range_ids_raise(gpu):
     with pytest.raises(IndexError):
         prog.run(bad)
     np.testing.assert_array_equal(_logits(prog, m.inputs)["logits"], good)
+
+
+def test_compiled_fp32_keeps_the_attention_probabilities(gpu):
+    """With keep_values, read_value returns the attention probabilities of an fp32 program (they are not stored
+    otherwise): those of the stored q and k in float64, and the logits are those of the program without them."""
+    from hackathon_amd import models
+
+    m = models.build_decoder(precision="fp32", name="decoder", batch=2, seq=70, d_model=128, heads=2, ffn=256,
+                             layers=1, vocab=50)
+    plan, prog, weights = _compiled(m, "fp32", keep_values=True)
+    got = _logits(prog, m.inputs)["logits"]
+    scores = next(n for n in m.graph.nodes.values() if n.op_type == "FusedAttentionScores")
+    probs = prog.read_value(scores.outputs[0])
+    assert probs.shape == (2, 2, 70, 70) and not np.triu(probs, 1).any()
+    np.testing.assert_allclose(probs.sum(-1), 1.0, rtol=1e-5)
+    q, kt = (prog.read_value(i).astype(np.float64) for i in scores.inputs[:2])
+    s = q @ kt / 8.0 + np.triu(np.full((70, 70), -np.inf), 1)
+    e = np.exp(s - s.max(-1, keepdims=True))
+    np.testing.assert_allclose(probs, e / e.sum(-1, keepdims=True), rtol=1e-4, atol=1e-7)
+    np.testing.assert_array_equal(got, _logits(_compiled(models.build_decoder(
+        precision="fp32", name="decoder", batch=2, seq=70, d_model=128, heads=2, ffn=256, layers=1, vocab=50),
+        "fp32")[1], m.inputs)["logits"])
