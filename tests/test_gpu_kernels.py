@@ -260,6 +260,25 @@ def test_flash_attention_host_checks(gpu):
         _lib.launch(a, None)
 
 
+def test_flash_attention_fp32_host_checks(gpu):
+    """Calls that the fp32 kernel cannot take are refused before any launch."""
+    from hackathon_amd import _lib
+    from hackathon_amd.device import DeviceArray
+
+    buf = DeviceArray.empty((16 * 64 + 4,), np.float32)
+    ok = dict(q=buf.ptr, k=buf.ptr, v=buf.ptr, out=buf.ptr, batch=1, heads=1, seq_q=16, seq_k=16, head_dim=64,
+              dtype=_lib.F32, q_ss=64, k_ss=64, v_ss=64, o_ss=64, scale=0.125, mask_kind=0)
+    for bad, match in [(dict(dtype=_lib.F16), "fp32"), (dict(head_dim=32), "head_dim"), (dict(seq_k=0), "sizes"),
+                       (dict(heads=0), "sizes"), (dict(mask_kind=3), "mask_kind"), (dict(mask_kind=2), "mask"),
+                       (dict(k_ss=66), "multiples of 4"), (dict(o_sh=1), "multiples of 4"),
+                       (dict(v=buf.ptr + 4), "misaligned"), (dict(out=buf.ptr + 8), "misaligned")]:
+        a = _lib.FlashF32Args()
+        for name, value in {**ok, **bad}.items():
+            setattr(a, name, value)
+        with pytest.raises(_lib.C3HError, match=match):
+            _lib.launch(a)
+
+
 @pytest.mark.parametrize("kind", ["fp16", "bf16"])
 @pytest.mark.parametrize("mask_kind", [0, 1, 2])
 @pytest.mark.parametrize("b,h,s", [(2, 3, 64), (1, 2, 200), (2, 1, 256),
@@ -1065,8 +1084,10 @@ def test_qgemm_big_tile_matches_128_tiles(gpu, m, n, k, mode, act):
 @pytest.mark.parametrize("m,n,k,mode,act,act_kind,switch,qscale", [
     (4096, 4096, 256, 3, 2, "bf16", None, 0.0417),                  # 256x256 tile, GELU in registers
     (4096, 4096, 256, 3, 2, "bf16", "C3H_DISABLE_BIGTILE", 0.0417), # 128x128 DMA tile, staged GELU epilogue
-    (300, 200, 256, 3, 1, "fp16", None, 0.0417),                    # 128x128, direct epilogue
-    (300, 70, 256, 2, 0, "fp32", None, 0.0417),                     # unaligned rows: staged, partial stores
+    (300, 200, 256, 3, 1, "fp16", None, 0.0417),                    # 32x32 tiles
+    (300, 200, 256, 3, 1, "fp16", "C3H_DISABLE_SMALLTILE", 0.0417), # 128x128, direct epilogue
+    (300, 70, 256, 2, 0, "fp32", None, 0.0417),                     # 16x32 tiles, unaligned rows
+    (300, 70, 256, 2, 0, "fp32", "C3H_DISABLE_SMALLTILE", 0.0417),  # unaligned rows: staged, partial stores
     (300, 200, 256, 3, 2, "bf16", "C3H_DISABLE_DMA", 0.0417),       # register-prefetch kernel
     (16384, 3072, 768, 3, 2, "bf16", None, 0.0417),                 # W8A8 FFN1
     (4096, 4096, 256, 2, 1, "bf16", None, 0.06),                    # multiplier fp32(1 / 0.06) - 1 ulp
@@ -1558,6 +1579,11 @@ def test_layernorm_int8_output_equals_layernorm_then_quantize(gpu, rows, cols, d
 _with_env = switches.with_switch
 
 
+def _shared_tiles(run):
+    """run() with the 128- and 256-row tiles on every shape, instead of the small and the 64-column ones."""
+    return _with_env("C3H_DISABLE_SMALLTILE", "1", run)
+
+
 @pytest.mark.parametrize("kind", ["bf16", "fp16", "int8"])
 @pytest.mark.parametrize("m,n,k", [(300, 200, 64), (256, 128, 128), (130, 70, 192), (1000, 256, 320),
                                    (4096, 512, 1152), (512, 64, 576), (2048, 2048, 512)])
@@ -1601,10 +1627,10 @@ def test_gemm_register_pipelined_matches_two_stage(gpu, kind, m, n, k):
         return out.get().copy()
 
     print(f"register pipelining {kind} {m}x{n}x{k}", flush=True)
-    want = _with_env("C3H_DISABLE_BIGTILE", "1", lambda: _with_env("C3H_DMA_RP", "0", run))
+    want = _with_env("C3H_DISABLE_BIGTILE", "1", lambda: _shared_tiles(lambda: _with_env("C3H_DMA_RP", "0", run)))
     assert np.any(want.view(np.uint8) != 0)
     for rp in ("2", "3", "4"):
-        got = _with_env("C3H_DISABLE_BIGTILE", "1", lambda: _with_env("C3H_DMA_RP", rp, run))
+        got = _with_env("C3H_DISABLE_BIGTILE", "1", lambda: _shared_tiles(lambda: _with_env("C3H_DMA_RP", rp, run)))
         np.testing.assert_array_equal(got.view(np.uint8), want.view(np.uint8), err_msg=f"RP stages {rp}")
 
 
@@ -1644,10 +1670,10 @@ def test_conv_register_pipelined_matches_two_stage(gpu, n, hw, c, o, kh, stride)
         return out.get().copy()
 
     print(f"register pipelining conv n={n} {hw}x{hw} c={c} o={o} k={kh} s={stride}", flush=True)
-    want = _with_env("C3H_DISABLE_BIGTILE", "1", lambda: _with_env("C3H_DMA_RP", "0", run))
+    want = _with_env("C3H_DISABLE_BIGTILE", "1", lambda: _shared_tiles(lambda: _with_env("C3H_DMA_RP", "0", run)))
     assert np.any(want.view(np.uint8) != 0)
     for rp in ("2", "3", "4"):
-        got = _with_env("C3H_DISABLE_BIGTILE", "1", lambda: _with_env("C3H_DMA_RP", rp, run))
+        got = _with_env("C3H_DISABLE_BIGTILE", "1", lambda: _shared_tiles(lambda: _with_env("C3H_DMA_RP", rp, run)))
         np.testing.assert_array_equal(got.view(np.uint8), want.view(np.uint8), err_msg=f"RP stages {rp}")
 
 
@@ -1890,6 +1916,142 @@ def test_small_output_conv_matches_the_general_kernel(gpu, kind, c, n, hw, o, ks
             assert np.all(np.abs(got.astype(np.float64) - want) <= 2 * k * k * 2.0 ** -23 + 2.0 ** -22 * np.abs(want))
         else:
             np.testing.assert_array_equal(got.view(np.uint16), want.view(np.uint16), err_msg=switch)
+
+
+@pytest.mark.parametrize("kind", ["bf16", "fp16", "int8", "fp8"])
+@pytest.mark.parametrize("m,n,k,form", [
+    (1000, 1032, 192, "relu"), (1011, 1030, 80, "program"), (1000, 1032, 320, "gelu"),    # 64 x 64 tiles
+    (1900, 2056, 192, "gelu"), (1901, 2050, 64, "relu"), (1900, 2056, 96, "program"),     # 128 x 64
+    (2100, 2504, 64, "relu")])                                   # 128 x 64 past one 128 x 128 tile per CU
+def test_mid_tile_gemm_matches_the_128_tiles(gpu, kind, m, n, k, form):
+    """The 64-column DMA tiles sum K in the order of the 128 x 128 ones: the same bits, at ragged M and N (rows
+    too short for whole vectors among them), with the register and the staged epilogue and both kinds of output
+    (16-bit and fp32; int8 codes and bf16)."""
+    from hackathon_amd import _lib
+    from hackathon_amd.c35 import engine as E
+    from hackathon_amd.device import BF16, DeviceArray
+
+    rng = np.random.default_rng(m + n + k)
+    if kind == "fp8":
+        a, b = (rng.integers(0, 0x40, s, dtype=np.uint8) | (rng.integers(0, 2, s, dtype=np.uint8) << 7) for s in
+                ((m, k), (n, k)))
+    elif kind == "int8":
+        a, b = (rng.integers(-128, 128, s, dtype=np.int8) for s in ((m, k), (n, k)))
+    else:
+        a, b = (_bits(rng.standard_normal(s, dtype=np.float32), kind)[0] for s in ((m, k), (n, k)))
+    ad, bd, bias = _dev(a), _dev(b), _dev(rng.standard_normal(n, dtype=np.float32))
+    scale = _dev(rng.random(max(m, n), dtype=np.float32) + 0.5)
+    prog = [(_lib.EW_MUL, 0, 2, 0.0), (_lib.EW_ADD, 1, 0, 0.0)]
+    kw = {"relu": dict(act=1), "gelu": dict(act=2, imm=[math.sqrt(2.0), 1.0, 0.5]),
+          "program": dict(program=prog, imm=[0.25])}[form]
+    types = {"int8": ((np.int8, _lib.I8), (BF16, _lib.BF16)), "fp8": ((np.float16, _lib.F16), (np.float32, _lib.F32)),
+             "bf16": ((BF16, _lib.BF16), (np.float32, _lib.F32)), "fp16": ((np.float16, _lib.F16), (np.float32, _lib.F32))}
+
+    def run(np_type, code):
+        out = DeviceArray.from_host(np.zeros((m, n), np_type))
+        g = {"fp8": _lib.Fp8GemmArgs, "int8": _lib.QGemmArgs}.get(kind, _lib.GemmArgs)()
+        g.a, g.b, g.out, g.m, g.n, g.k, g.lda, g.ldb, g.ldo = ad.ptr, bd.ptr, out.ptr, m, n, k, k, k, n
+        g.out_dtype, g.epi = code, E.epilogue(bias=bias, bias_mode=2, **kw)
+        if kind == "fp8":
+            g.a_scale, g.b_scale = scale.ptr, scale.ptr
+        elif kind == "int8":
+            g.a_scale, g.y_scale, g.b_scale, g.mode = 0.02, 0.05, scale.ptr, 2
+            g.act_dtype, g.q_scale, g.q_zero = (_lib.BF16, 7.0, 3) if code == _lib.I8 else (0, 0.0, 0)
+        else:
+            g.batch, g.trans_b, g.in_dtype = 1, 1, ad.code
+        _lib.launch(g)
+        return out.get().view(np.uint8)
+
+    for np_type, code in types[kind]:
+        print(f"mid tile {kind} {m}x{n}x{k} {form} out {code}", flush=True)
+        got, want = run(np_type, code), _shared_tiles(lambda: run(np_type, code))
+        assert want.any()
+        np.testing.assert_array_equal(got, want)
+
+
+@pytest.mark.parametrize("kind", ["bf16", "fp16"])
+@pytest.mark.parametrize("n,hw,c,o,stride", [(20, 28, 64, 100, 1), (37, 28, 64, 128, 1), (21, 56, 64, 128, 2)])
+def test_mid_tile_conv_matches_the_128_tiles(gpu, kind, n, hw, c, o, stride):
+    """3x3 convs on the 64-column DMA tiles (64 x 64 and 128 x 64, ragged output channels, stride 2) give the
+    bits of the 128-row tiles."""
+    from hackathon_amd import _lib
+    from hackathon_amd.c35 import engine as E
+    from hackathon_amd.device import DeviceArray
+
+    rng = np.random.default_rng(n + hw + o)
+    ho = (hw - 1) // stride + 1
+    x, w, res = (_dev(_bits(rng.standard_normal(s, dtype=np.float32), kind)[0]) for s in
+                 ((n, hw, hw, c), (o, 3, 3, c), (n, ho, ho, o)))
+    bias = _dev(rng.standard_normal(o, dtype=np.float32))
+
+    def run():
+        out = DeviceArray.from_host(np.zeros((n, ho, ho, o), x.dtype))
+        a = _lib.ConvArgs()
+        a.x, a.w, a.out = x.ptr, w.ptr, out.ptr
+        a.n, a.c, a.h, a.w_, a.c_stride, a.c_pack, a.o, a.kh, a.kw, a.sh, a.sw = n, c, hw, hw, c, c, o, 3, 3, stride, stride
+        a.pad_top, a.pad_left, a.dh, a.dw, a.ho, a.wo = 1, 1, 1, 1, ho, ho
+        a.out_layout, a.in_dtype, a.out_dtype = 1, x.code, x.code
+        a.epi = E.epilogue(bias=bias, bias_mode=2, act=1, residual=res)
+        print(f"mid conv {kind} n={n} {hw} {c}->{o} stride {stride}", flush=True)
+        _lib.launch(a)
+        return out.get().view(np.uint16)
+
+    got, want = run(), _shared_tiles(run)
+    assert want.any()
+    np.testing.assert_array_equal(got, want)
+
+
+@pytest.mark.parametrize("kind,n,hw,o,c,c_pack,c_stride,dil", [
+    *((kind, *case) for kind in ("fp32", "bf16") for case in [
+        (1, 9, 72, 64, 64, 96, 1), (1, 9, 72, 64, 64, 64, 2), (2, 11, 72, 40, 64, 64, 2),  # small tiles
+        (20, 28, 128, 64, 64, 72, 2)]),                                                    # 64-row tiles
+    ("fp32", 1, 9, 72, 40, 64, 40, 1)])                                                    # packed channels past the pixel
+def test_conv_dilation_and_channel_strides(gpu, kind, n, hw, o, c, c_pack, c_stride, dil):
+    """3x3 convs with dilation, pixels further apart than their channels, and weights padded to more channels
+    than the input has, in whole K tiles of one tap, against float64 (K 2^-24 of sum |a b| for the fp32 sums,
+    plus half an ulp of a 16-bit output).  Where the weights have more channels than a pixel, an infinity in
+    one pixel reaches only the outputs whose window holds it: the padding is not multiplied with the next pixel."""
+    from hackathon_amd import _lib
+    from hackathon_amd.c35 import engine as E
+    from hackathon_amd.device import DeviceArray
+
+    rng = np.random.default_rng(n + hw + o + c_stride + dil)
+    rounded = (lambda v: (v, v)) if kind == "fp32" else (lambda v: _bits(v, kind))
+    x = np.zeros((n, hw, hw, c_stride), np.float32)
+    x[..., :c] = rng.standard_normal((n, hw, hw, c), dtype=np.float32)
+    w = np.zeros((o, 3, 3, c_pack), np.float32)
+    w[..., :c] = rng.standard_normal((o, 3, 3, c), dtype=np.float32)
+    if c_stride < c_pack:
+        x[0, 4, 4, 3] = np.inf
+    (xs, x), (ws, w) = rounded(x), rounded(w)
+    bias = rng.standard_normal(o, dtype=np.float32)
+    xd, wd, bd = _dev(xs), _dev(ws), _dev(bias)
+    out = DeviceArray.empty((n, hw, hw, o), xd.dtype)
+    a = _lib.ConvArgs()
+    a.x, a.w, a.out = xd.ptr, wd.ptr, out.ptr
+    a.n, a.c, a.h, a.w_, a.c_stride, a.c_pack, a.o, a.kh, a.kw, a.sh, a.sw = n, c, hw, hw, c_stride, c_pack, o, 3, 3, 1, 1
+    a.pad_top, a.pad_left, a.dh, a.dw, a.ho, a.wo = dil, dil, dil, dil, hw, hw
+    a.out_layout, a.in_dtype, a.out_dtype = 1, xd.code, xd.code
+    a.epi = E.epilogue(bias=bd, bias_mode=2)
+    print(f"conv {kind} n={n} {hw} c={c}/{c_pack}/{c_stride} dilation {dil}", flush=True)
+    _lib.launch(a)
+    got = (out.get() if kind == "fp32" else _from16(out.get(), kind)).reshape(n, hw, hw, o).astype(np.float64)
+    xp = np.zeros((n, hw + 2 * dil, hw + 2 * dil, c))
+    xp[:, dil:dil + hw, dil:dil + hw] = x[..., :c].reshape(n, hw, hw, c)
+    ref, size = np.zeros((n, hw, hw, o)), np.zeros((n, hw, hw, o))
+    hit = np.zeros((n, hw, hw), bool)
+    for i in range(3):
+        for j in range(3):
+            win = xp[:, i * dil:i * dil + hw, j * dil:j * dil + hw]
+            hit |= np.isinf(win).any(-1)
+            win = np.where(np.isinf(win), 0.0, win)
+            wt = w.reshape(o, 3, 3, c_pack)[:, i, j, :c].T.astype(np.float64)
+            ref += win @ wt
+            size += np.abs(win) @ np.abs(wt)
+    ref += bias
+    bound = (9 * c + 8) * 2.0 ** -24 * (size + np.abs(bias)) + (0 if kind == "fp32" else 2.0 ** -8 * np.abs(ref))
+    assert hit.any() == (c_stride < c_pack)
+    assert np.all((np.abs(got - ref) <= bound) | hit[..., None]) and not np.isfinite(got[hit]).any()
 
 
 @pytest.mark.parametrize("mask_kind", [0, 1, 2])
