@@ -2,7 +2,9 @@
 // split-K, int8, fp8 and W4A16 GEMM).  The kernels and launch templates
 // live in gemm_kernels.h; the per-type launchers are instantiated in
 // gemm_bf16.hip, gemm_bf16_conv.hip, gemm_f16.hip, gemm_f16_conv.hip,
-// gemm_i8.hip, gemm_f8.hip, gemm_w4.hip and gemm_f32.hip.
+// gemm_i8.hip, gemm_f8.hip, gemm_w4.hip and gemm_f32.hip, those of the
+// small-output kernels (gemm_ks.h) in gemm_ks_16.hip and gemm_ks_8.hip (int8,
+// E4M3 and fp32), of the 64-column tiles in gemm_mid_16.hip and gemm_mid_8.hip.
 #include <stdlib.h>
 #include <mutex>
 
