@@ -275,8 +275,8 @@ struct Problem {
   // E8M0 exponents [n][ldbs] of its 32-element blocks (bs_bytes in all)
   const uint8_t* b_blk;
   int64_t ldbs, bs_bytes;
-  int k_part;  // K of each partial sum of a split-K GEMM run in one launch
   c3h_epilogue epi;
+  int k_part;  // K of each partial sum of a split-K GEMM run in one launch
 };
 
 enum AMode { kDenseK = 0, kDenseM = 1, kConv = 2 };
@@ -2841,24 +2841,30 @@ int launch_w4_tile(Problem p, hipStream_t s) {
 }
 // 64 x 64 tiles up to three per CU, then 128 x 64 up to 1.5 tiles of 128 x 128
 // per CU and, where K is at most 1024, between 2 and 2.5 of them: 128 x 128
-// runs two blocks per CU, and its last round would be nearly empty.  From
-// there on 128 x 128, which widens each weight for twice the rows.  Measured (M
-// x N x K, us, 128 x 128 / 128 x 64 / 64 x 64): 333 x 512 x 2048 27.1 / 20.2 /
-// 16.3, 4000 x 768 x 3072 (756 tiles of 64 x 64) 44.0 / 40.2 / 38.0, 2048 x
-// 2048 x 512 (1024) 11.3 / 10.9 / 11.7, 8000 x 512 x 2048 (1000) 31.4 / 29.2 /
-// 32.4; 3000 x 2048 x 512 (384 tiles of 128 x 128) 17.0 / 14.4 / 16.7, 8000 x
-// 1000 x 512 (504) 18.0 / 20.4 / 19.7, 6000 x 1536 x 512 (564) 24.2 / 21.0 /
-// 23.2, 13000 x 768 x 768 (612) 29.7 / 27.4 / 32.6, 7000 x 1536 x 512 (660)
-// 23.0 / 23.8 / 26.0, 15000 x 768 x 768 (708) 30.0 / 32.0 / 37.7, 16384 x 1536
-// x 512 (1536) 43.1 / 46.3 / 58.0, 16384 x 8192 x 512 (8192) 189 / 210 / 260.
-// Every tile sums K in the same order.
+// runs two blocks per CU, and its last round would be nearly empty. From there
+// on 128 x 128, which widens each weight for twice the rows -- but with GELU
+// 128 x 64 at any number past 2: its VALU epilogue is then the longer part,
+// and smaller blocks overlap it better with their neighbours' loops. Every
+// tile sums K in the same order.
+//
+// Measured (M x N x K, us, 128 x 128 / 128 x 64 / 64 x 64): 333 x 512 x 2048
+// 27.1 / 20.2 / 16.3, 4000 x 768 x 3072 (756 tiles of 64 x 64) 44.0 / 40.2 /
+// 38.0, 2048 x 2048 x 512 (1024) 11.3 / 10.9 / 11.7, 8000 x 512 x 2048 (1000)
+// 31.4 / 29.2 / 32.4; 3000 x 2048 x 512 (384 tiles of 128 x 128) 17.0 / 14.4 /
+// 16.7, 8000 x 1000 x 512 (504) 18.0 / 20.4 / 19.7, 6000 x 1536 x 512 (564)
+// 24.2 / 21.0 / 23.2, 13000 x 768 x 768 (612) 29.7 / 27.4 / 32.6, 7000 x 1536
+// x 512 (660) 23.0 / 23.8 / 26.0, 15000 x 768 x 768 (708) 30.0 / 32.0 / 37.7,
+// 16384 x 1536 x 512 (1536) 43.1 / 46.3 / 58.0, 16384 x 8192 x 512 (8192) 189
+// / 210 / 260. GELU: 16384 x 512 x 512 (512) 23.1 / 23.9, 6000 x 3072 x 768
+// (1128) 62.3 / 53.6, 12000 x 2048 x 512 (1504) 58.9 / 55.8, 16384 x 2048 x
+// 512 (2048) 79.3 / 74.2, 16384 x 3072 x 768 (3072) 133.8 / 134.6.
 template <typename TO>
 int launch_w4(Problem p, hipStream_t s) {
   const int64_t cus = device_cus(), tiles128 = ceil_div(p.m, 128) * ceil_div(p.n, 128);
   if (ceil_div(p.m, 64) * ceil_div(p.n, 64) <= 3 * cus) return launch_w4_tile<TO, 64, 64, 4, 1>(p, s);
   if (p.n <= 64) return launch_w4_tile<TO, 256, 64, 4, 1>(p, s);
-  if (2 * tiles128 <= 3 * cus || (p.k <= 1024 && tiles128 > 2 * cus && 2 * tiles128 <= 5 * cus))
-    return launch_w4_tile<TO, 128, 64, 4, 1>(p, s);
+  const bool short_k = p.k <= 1024 && tiles128 > 2 * cus && (p.epi.act == 2 || 2 * tiles128 <= 5 * cus);
+  if (2 * tiles128 <= 3 * cus || short_k) return launch_w4_tile<TO, 128, 64, 4, 1>(p, s);
   return launch_w4_tile<TO, 128, 128, 2, 2>(p, s);
 }
 
