@@ -112,9 +112,9 @@ namespace {
 // 64 x 64 leaves the fewest CUs idle.  Against the register-staged kernel
 // below (its k-major LDS tiles took four scalar LDS stores per load and a
 // scalar read per MFMA operand): 3x3 convs of a batch of 256, 128 channels
-// 16 x 16 220 -> 160 us (121 TFLOP/s; a pure MFMA loop reaches 151), 512
-// channels 4 x 4 274 -> 169 us; dense 2048 x 2048 x 512 75 -> 40 us,
-// 2048 x 512 x 512 28 -> 15 us.
+// 16 x 16 220 -> 159 us (121 TFLOP/s repeated alone, 115 among the model's
+// other launches; a pure MFMA loop reaches 151), 512 channels 4 x 4 274 -> 161
+// us; dense 2048 x 8192 x 512 142 us, 2048 x 512 x 512 28 -> 13 us.
 template <int AM>
 int launch_f32_dma(Problem p, hipStream_t s) {
   dim3 grid;
